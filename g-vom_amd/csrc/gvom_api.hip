@@ -53,7 +53,7 @@ constexpr int64_t NOALLOC_POINTS = 131072;
 
 struct ScratchLayout {
     int64_t world, valid, k0, v0, k1, v1, hist, hwords, blk, blk_words, seg_key, seg_start, mom, part, rsec,
-        rorder, total;
+        rorder, azhist, azwords, total;
 };
 
 constexpr int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
@@ -77,6 +77,8 @@ constexpr ScratchLayout scratch_layout(int64_t n) {
     L.part = at;      at = align256(at + n * (int64_t)sizeof(Moment));
     L.rsec = at;      at = align256(at + n);
     L.rorder = at;    at = align256(at + n * 4);
+    L.azwords = gvom_plan::alloc_az_hist_words(n);
+    L.azhist = at;    at = align256(at + L.azwords * 4);
     L.total = at;
     return L;
 }
@@ -221,11 +223,16 @@ struct gvom_handle {
     std::vector<hipEvent_t> ev_pool;
     std::vector<int> set_used;   // bit k set when event k of that set was recorded
     int cur_set = -1;
+    // azimuth-ordered cast for scans it pays for (gvom_plan::az_pays); the settings below apply
+    // to the others, or to all when it is off
+    int ray_az = 1;
     int ray_block = 128, ray_rpt = 1, ray_box = 0, ray_xcd = 0, ray_spread = 1;
     int64_t ray_stride = 0;   // gvom_set_ray_rings: points per ring (0: linear ray order)
     int ray_patch = 0;        // rings per patch
     uint8_t *rsec = nullptr;
     uint32_t *rorder = nullptr;
+    uint32_t *azhist = nullptr;   // azimuth bin counts (az_rows); zero between scan stages
+    int64_t azwords = 0;
     int8_t *grids = nullptr;   // OccupancyGrid payloads staged for host copies (5 * X bytes)
     uint8_t *raw = nullptr;    // PointCloud2 bytes staged from the host
     int64_t rawcap = 0;
@@ -284,7 +291,7 @@ static void free_all(gvom_handle *h) {
                     h->slope_x, h->slope_y, h->maps_block, h->delta, h->occ_list,
                     h->col_count, h->chunk_tot, h->export_buf, h->pts_in, h->world, h->valid, h->k0, h->v0, h->k1, h->v1,
                     h->hist, h->blk, h->seg_key, h->seg_start, h->mom, h->part, h->sd, h->diff_rec,
-                    h->diff_colh, h->diff_part, h->diff_sums, h->diff_colpt, h->diff_pmark, h->graph_sd, h->rsec, h->rorder, h->grids, h->raw, h->tscratch,
+                    h->diff_colh, h->diff_part, h->diff_sums, h->diff_colpt, h->diff_pmark, h->graph_sd, h->rsec, h->rorder, h->azhist, h->grids, h->raw, h->tscratch,
                     h->occ_bits, h->zero_page};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -461,6 +468,8 @@ extern "C" void *gvom_stream(gvom_handle *h) {
     return (void *)h->stream;
 }
 
+static hipError_t mark_back(gvom_handle *h);
+
 // Grow per-batch work buffers (points) and per-slot record capacity (cells per scan).
 static int ensure_capacity(gvom_handle *h, int64_t max_scan, int64_t batch_pts) {
     const Geo &g = h->g;
@@ -508,7 +517,7 @@ static int ensure_capacity(gvom_handle *h, int64_t max_scan, int64_t batch_pts) 
         void **ptrs[] = {(void **)&h->pts_in, (void **)&h->world, (void **)&h->valid, (void **)&h->k0,
                          (void **)&h->v0, (void **)&h->k1, (void **)&h->v1, (void **)&h->hist, (void **)&h->blk,
                          (void **)&h->seg_key, (void **)&h->seg_start, (void **)&h->mom, (void **)&h->part,
-                         (void **)&h->rsec, (void **)&h->rorder};
+                         (void **)&h->rsec, (void **)&h->rorder, (void **)&h->azhist};
         for (void **q : ptrs) {
             void *old = *q;
             *q = nullptr;
@@ -533,6 +542,10 @@ static int ensure_capacity(gvom_handle *h, int64_t max_scan, int64_t batch_pts) 
         CKH(h, dalloc(&h->part, pc));
         CKH(h, dalloc(&h->rsec, pc));
         CKH(h, dalloc(&h->rorder, pc));
+        h->azwords = gvom_plan::alloc_az_hist_words(pc);
+        CKH(h, dalloc(&h->azhist, h->azwords));
+        CKH(h, launch_fill_i32((int32_t *)h->azhist, 0, h->azwords, h->stream));
+        CKH(h, mark_back(h));   // an overlapped scan stage follows the fill
         h->ptcap = pc;
     }
     return GVOM_OK;
@@ -631,8 +644,10 @@ struct WorkBufs {
     Moment *mom = nullptr, *part = nullptr;
     uint8_t *rsec = nullptr;
     uint32_t *rorder = nullptr;
+    uint32_t *azhist = nullptr;
+    int64_t azwords = 0;
     int64_t cap = 0;          // points
-    bool clear_hist = false;  // zero the first histogram before the transform kernel counts into it
+    bool clear_hist = false;  // zero the counts that the transform kernel adds to
 };
 
 static WorkBufs scratch_bufs(uint8_t *base) {
@@ -654,6 +669,8 @@ static WorkBufs scratch_bufs(uint8_t *base) {
     w.part = (Moment *)(base + L.part);
     w.rsec = base + L.rsec;
     w.rorder = (uint32_t *)(base + L.rorder);
+    w.azhist = (uint32_t *)(base + L.azhist);
+    w.azwords = L.azwords;
     w.cap = NOALLOC_POINTS;
     w.clear_hist = true;   // another call may have left the shared histogram dirty
     return w;
@@ -678,6 +695,8 @@ static WorkBufs handle_bufs(gvom_handle *h) {
     w.part = h->part;
     w.rsec = h->rsec;
     w.rorder = h->rorder;
+    w.azhist = h->azhist;
+    w.azwords = h->azwords;
     w.cap = h->ptcap;
     return w;
 }
@@ -754,7 +773,7 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     }
     const WorkBufs W = scratch ? *scratch : handle_bufs(h);
     if (!h->slot_recs || !W.world || !W.valid || !W.k0 || !W.v0 || !W.k1 || !W.v1 || !W.hist || !W.blk ||
-        !W.seg_key || !W.seg_start || !W.mom || !W.part || !W.rsec || !W.rorder || W.cap < NT || W.cap < 1 ||
+        !W.seg_key || !W.seg_start || !W.mom || !W.part || !W.rsec || !W.rorder || !W.azhist || W.cap < NT || W.cap < 1 ||
         (!on_device && !W.pts_in)) {
         h->err = "internal: work buffers not allocated";
         return GVOM_ESTATE;
@@ -780,7 +799,8 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     }
     // without allocation, a handle whose tiled scratch does not exist yet casts directly
     // (same counts)
-    const bool tiled = cast && h->ray_tiled != 0 && tiled_fits(g) && (!scratch || h->tscratch);
+    const bool az = cast && h->ray_az != 0 && gvom_plan::az_pays(NT, g.XY);
+    const bool tiled = cast && !az && h->ray_tiled != 0 && tiled_fits(g) && (!scratch || h->tscratch);
     if (tiled) {
         int rc_t = ensure_tile_scratch(h);
         if (h->buf_gen != gen0) h->diff_n = -1;
@@ -843,11 +863,15 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     }
     h->diff_n = -1;   // every check passed: the work buffers a pending gvom_diff_backward reads are reused below
     stage_event(h, 0, fs);
-    const bool xcd = cast && h->ray_xcd != 0;
+    const bool xcd = cast && !az && h->ray_xcd != 0;
     if (xcd) CKH(h, launch_fill_i32(&h->st->sec_count[0], 0, 16, fs));   // sec_count and sec_cursor
-    if (W.clear_hist) CKH(h, launch_fill_i32((int32_t *)W.hist, 0, W.hwords, fs));
+    if (W.clear_hist) {
+        CKH(h, launch_fill_i32((int32_t *)W.hist, 0, W.hwords, fs));
+        if (az) CKH(h, launch_fill_i32((int32_t *)W.azhist, 0, gvom_plan::az_hist_words(NT, S), fs));
+    }
     CKH(h, launch_prepare(dtype, pts, W.world, W.k0, W.v0, W.valid, sd, S, NT, g, h->st,
-                          xcd ? W.rsec : nullptr, W.hist, W.hwords, fs));
+                          xcd ? RAY_SECTORS : (az ? RAY_AZIMUTH : RAY_LINEAR), W.rsec, W.hist, W.hwords, W.azhist,
+                          W.azwords, fs));
     if (xcd) CKH(h, launch_ray_order(W.rsec, NT, h->st, W.rorder, fs));
     // fork: keys, segments and chunk partials on the side stream, concurrent with the cast
     CKH(h, hipEventRecord(h->ev_fork, fs));
@@ -858,11 +882,17 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     CKH(h, launch_segments(dtype, W.world, sk, sv, NT, sd, S, g, h->st, W.hist, W.hwords, W.blk, W.blk_words,
                            W.seg_start, W.seg_key, W.part, h->side));
     CKH(h, hipEventRecord(h->ev_join, h->side));
-    // the tiled path's conversion writes every word of the slot tables; the direct cast counts
+    // the tiled path's conversion writes every word of the slot tables; the direct casts count
     // into cleared tables, cleared here, beside the sort chain (nothing before the cast reads them)
-    if (!tiled) CKH(h, launch_clear_slots(h->slot_tables, h->st, S, g, fs));
+    if (az)
+        CKH(h, launch_az_order(W.rsec, W.valid, sd, S, NT, g, h->st, W.azhist, W.azwords, W.rorder, h->slot_tables,
+                               h->slot_table_words, -1, fs));
+    else if (!tiled) CKH(h, launch_clear_slots(h->slot_tables, h->st, S, g, fs));
     stage_event(h, 1, fs);
-    if (cast)
+    if (az)
+        CKH(h, launch_raycast_az(dtype, W.world, sd, S, NT, g, h->st, h->slot_tables, h->slot_table_words, W.rorder,
+                                 W.azhist, W.azwords, 1, -1, fs));
+    else if (cast)
         CKH(h, launch_raycast(dtype, W.world, W.valid, sd, S, NT, g, h->st, tiled ? h->tscratch : h->slot_tables,
                               tiled ? h->tscratch_words : h->slot_table_words,
                               h->ray_block, h->ray_rpt, tiled ? 0 : h->ray_box, tiled ? 1 : 0, -1,
@@ -2036,7 +2066,7 @@ extern "C" int gvom_autotune(gvom_handle *h, const void *points, int64_t n, int3
     int32_t *scratch = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int out = GVOM_OK;
-    int bb = h->ray_block, br = h->ray_rpt, bx = h->ray_box, bo = h->ray_xcd, bt = h->ray_tiled;
+    int bb = h->ray_block, br = h->ray_rpt, bx = h->ray_box, bo = h->ray_xcd, bt = h->ray_tiled, ba = 0;
     float best = 1e30f;
     do {
         const bool can_tile = tiled_fits(g);
@@ -2053,9 +2083,8 @@ extern "C" int gvom_autotune(gvom_handle *h, const void *points, int64_t n, int3
         if (hipMemcpyAsync(saved, h->st, sizeof(DevState), hipMemcpyDeviceToDevice, st) != hipSuccess ||
             hipMemcpyAsync(h->sd, &d, sizeof(ScanDesc), hipMemcpyHostToDevice, st) != hipSuccess ||
             launch_fill_i32(&h->st->sec_count[0], 0, 16, st) != hipSuccess ||
-            launch_prepare(dtype, points, h->world, h->k0, h->v0, h->valid, h->sd, 1, n, g, h->st, h->rsec, nullptr, 0,
-                           st) !=
-                hipSuccess ||
+            launch_prepare(dtype, points, h->world, h->k0, h->v0, h->valid, h->sd, 1, n, g, h->st, RAY_SECTORS, h->rsec,
+                           nullptr, 0, nullptr, 0, st) != hipSuccess ||
             launch_ray_order(h->rsec, n, h->st, h->rorder, st) != hipSuccess) {
             h->err = "autotune: setup failed";
             out = GVOM_EHIP;
@@ -2101,6 +2130,39 @@ extern "C" int gvom_autotune(gvom_handle *h, const void *points, int64_t n, int3
                         bt = itile;
                     }
                 }
+        // the azimuth order, its grouping and the table clear included
+        const bool try_az = gvom_plan::az_pays(n, g.XY);
+        if (out == GVOM_OK && try_az &&
+            launch_prepare(dtype, points, h->world, h->k0, h->v0, h->valid, h->sd, 1, n, g, h->st, RAY_AZIMUTH, h->rsec,
+                           nullptr, 0, h->azhist, h->azwords, st) != hipSuccess) {
+            h->err = "autotune: setup failed";
+            out = GVOM_EHIP;
+        }
+        float t_az = 1e30f;
+        for (int rep = 0; rep < 3 && try_az && out == GVOM_OK; ++rep) {
+            float t = 0.f;
+            const bool ok = hipEventRecord(e0, st) == hipSuccess &&
+                            launch_az_order(h->rsec, h->valid, h->sd, 1, n, g, h->st, h->azhist, h->azwords, h->rorder,
+                                            scratch, g.V, 0, st) == hipSuccess &&
+                            launch_raycast_az(dtype, h->world, h->sd, 1, n, g, h->st, scratch, g.V, h->rorder,
+                                              h->azhist, h->azwords, 0, 0, st) == hipSuccess &&
+                            hipEventRecord(e1, st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
+                            hipEventElapsedTime(&t, e0, e1) == hipSuccess;
+            if (!ok) {
+                h->err = "autotune: timing run failed";
+                out = GVOM_EHIP;
+                break;
+            }
+            if (t < t_az) t_az = t;
+        }
+        if (out == GVOM_OK && t_az < best) {
+            best = t_az;
+            ba = 1;
+        }
+        if (launch_fill_i32((int32_t *)h->azhist, 0, h->azwords, st) != hipSuccess) {
+            h->err = "autotune: restoring state failed";
+            out = GVOM_EHIP;
+        }
         if (hipMemcpyAsync(h->st, saved, sizeof(DevState), hipMemcpyDeviceToDevice, st) != hipSuccess ||
             hipStreamSynchronize(st) != hipSuccess) {
             h->err = "autotune: restoring state failed";
@@ -2117,11 +2179,12 @@ extern "C" int gvom_autotune(gvom_handle *h, const void *points, int64_t n, int3
         h->ray_box = bx;
         h->ray_xcd = bo;
         h->ray_tiled = bt;
+        h->ray_az = ba;
         ++h->cfg_gen;
         if (chosen) {
             chosen[0] = bb;
             chosen[1] = br;
-            chosen[2] = bx | (bo << 1) | (bt << 2) | (h->ray_spread << 3);
+            chosen[2] = bx | (bo << 1) | (bt << 2) | (h->ray_spread << 3) | (ba << 4);
         }
         if (best_ms) *best_ms = best;
     }
@@ -2175,6 +2238,7 @@ extern "C" int gvom_set_raycast_config(gvom_handle *h, int32_t block, int32_t ra
         (flags & 1 && flags & 4))
         return GVOM_EINVAL;
     std::lock_guard<std::mutex> lk(h->mu);
+    h->ray_az = (flags >> 4) & 1;
     h->ray_block = block;
     h->ray_rpt = rays_per_thread;
     h->ray_box = flags & 1;

@@ -74,6 +74,7 @@ struct DevState {
     // set when a block gave up waiting for counts an earlier block publishes (PUB_READY
     // protocol; a defect): the state getters then report an error
     int32_t wait_fault;
+    int32_t ray_n[GVOM_MAX_BATCH];   // valid rays per scan of the batch in flight (k_az_order)
 };
 
 // Physical buffer of ring slot `slot`: the one holding its scan, and the one the scan stage in

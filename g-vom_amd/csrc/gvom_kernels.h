@@ -10,10 +10,25 @@ hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t s);
 // ---- scan stage (gvom_scan.hip) ------------------------------------------------------
 // Transform, validity, own-voxel sort key per point (reference gvom.py:1122-1163).
 // With hist (hwords words, radix_hist_entries): the sort's first-pass counts are accumulated
-// into hist, which must be zero.
+// into hist, which must be zero.  rmode: what rbin receives, RAY_SECTORS (8 azimuth sectors,
+// counted in st) or RAY_AZIMUTH (azimuth bins, counted in azhist, azwords words, which must be
+// zero).
+enum RayMode { RAY_LINEAR = 0, RAY_SECTORS = 1, RAY_AZIMUTH = 2 };
 hipError_t launch_prepare(int dtype, const void *in, void *world, uint32_t *keys, uint32_t *vals,
                           uint8_t *valid, const ScanDesc *sd, int S, int64_t NT, const Geo &g,
-                          DevState *st, uint8_t *rsec, uint32_t *hist, int64_t hwords, hipStream_t s);
+                          DevState *st, int rmode, uint8_t *rbin, uint32_t *hist, int64_t hwords, uint32_t *azhist,
+                          int64_t azwords, hipStream_t s);
+// Each scan's valid ray indices grouped by azimuth bin, in point order within a bin, from the
+// scan's first point's place in `order` on (st->ray_n = how many), and the S target slot
+// tables cleared, in one launch.  force_slot as for launch_raycast.
+hipError_t launch_az_order(const uint8_t *rbin, const uint8_t *valid, const ScanDesc *sd, int S, int64_t NT,
+                           const Geo &g, DevState *st, const uint32_t *azhist, int64_t azwords, uint32_t *order,
+                           int32_t *slot_tables, int64_t table_words, int force_slot, hipStream_t s);
+// The ray march over that order, counting in LDS, into the cleared slot tables; with
+// clear_counts the azimuth counts are zeroed for the next scan stage.
+hipError_t launch_raycast_az(int dtype, const void *world, const ScanDesc *sd, int S, int64_t NT, const Geo &g,
+                             const DevState *st, int32_t *slot_tables, int64_t table_words, const uint32_t *order,
+                             uint32_t *azhist, int64_t azwords, int clear_counts, int force_slot, hipStream_t s);
 // Tiled ray-cast scratch (4 x 4 x 1 voxels per 64-byte segment): words per scan, and the
 // conversion into the slot tables (which also zeroes the scratch).
 int64_t tile_scratch_words(const Geo &g);

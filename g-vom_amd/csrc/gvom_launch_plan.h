@@ -33,6 +33,22 @@ constexpr int64_t segment_flags_at(int64_t n) { return radix_scan_counts_at(n) +
 constexpr int64_t radix_hist_words(int64_t n) { return segment_flags_at(n) + blocks(n, SEG_TILE); }
 constexpr int64_t radix_hist_alloc_words(int64_t n) { return RADIX_HIST_SETS * radix_hist_words(n); }
 
+// ---- azimuth ray order: counts of AZ_BINS azimuth bins per (tile of RS_TILE points, scan) pair;
+// pair (t, s) has row t + s, so S scans over n points use blocks(n, RS_TILE) + S - 1 rows
+constexpr int AZ_BINS = 256;
+constexpr int64_t az_rows(int64_t n, int S) { return blocks(n, RS_TILE) + S - 1; }
+constexpr int64_t az_hist_words(int64_t n, int S) { return AZ_BINS * az_rows(n, S); }
+constexpr int64_t alloc_az_hist_words(int64_t n) { return az_hist_words(n, MAX_BATCH); }
+// The azimuth-ordered cast pays its grouping and its per-block set-up back on scans of at least
+// AZ_MIN_WORK points x map side (a bound of twice the ray steps).  Measured, grouping + cast +
+// table clear against the tiled cast + conversion (event-timed): 131,072 points on 256 x 256 x
+// 64 43 against 60 us, 235,877 on 512 x 512 x 64 90 against 125, 118,144 on 100 x 100 x 40 (12M)
+// 27 against 38; 62,256 on 256 x 256 x 64 (16M) 39 against 39; below the line 58,952 on 128 x
+// 128 x 32 (7.5M) 24 against 22, 51,830 on 151 x 151 x 100 (7.8M) 31 against 29, 7,763 on 64 x
+// 64 x 32 22 against 12.
+constexpr int64_t AZ_MIN_WORK = 12000000;
+constexpr bool az_pays(int64_t n, int32_t XY) { return n * XY >= AZ_MIN_WORK; }
+
 // ---- segment kernels: per block of SEG_TILE keys, W = 2 + 3 S counters (heads, valid keys,
 // then per scan of the batch in-map heads, halo heads, valid keys), plus one row of totals;
 // the C-ABI sizes the buffer for the largest batch

@@ -91,6 +91,22 @@ __device__ __forceinline__ int ray_sector(double dx, double dy) {
     return s < 0 ? 0 : (s > 7 ? 7 : s);
 }
 
+// Azimuth of a ray's xy direction in [0, 65536): monotone in the angle (the direction's position
+// along the unit diamond), without a trigonometric function.  Used only to order rays.
+__device__ __forceinline__ uint32_t ray_azimuth(float dx, float dy) {
+    const float sum = fabsf(dx) + fabsf(dy);
+    float q = sum > 0.0f ? dy / sum : 0.0f;   // [-1, 1]
+    if (dx < 0.0f) q = 2.0f - q;
+    else if (q < 0.0f) q = 4.0f + q;
+    const int k = (int)(q * 16384.0f);
+    return (uint32_t)(k < 0 ? 0 : (k > 65535 ? 65535 : k));
+}
+
+template <typename P>
+__device__ __forceinline__ uint32_t ray_azimuth_of(const ScanDesc &d, P x, P y) {
+    return ray_azimuth((float)((double)x - d.ego[0]), (float)((double)y - d.ego[1]));
+}
+
 // Radix sort tiles: RS_TILE keys per block of every pass.
 constexpr int RS_TILE = gvom_plan::RS_TILE;
 
@@ -104,14 +120,26 @@ __global__ __launch_bounds__(256) void k_prepare(const P *__restrict__ in, P *__
                                                  uint32_t *__restrict__ keys, uint32_t *__restrict__ vals,
                                                  uint8_t *__restrict__ valid,
                                                  const ScanDesc *__restrict__ sd, int S, int64_t NT,
-                                                 Geo g, DevState *__restrict__ st, uint8_t *__restrict__ rsec,
-                                                 uint32_t *__restrict__ hist, int64_t hwords) {
+                                                 Geo g, DevState *__restrict__ st, int rmode,
+                                                 uint8_t *__restrict__ rsec, uint32_t *__restrict__ hist,
+                                                 int64_t hwords, uint32_t *__restrict__ azhist) {
     __shared__ int32_t scount[8];
-    __shared__ uint32_t lh[256];
-    if (rsec && threadIdx.x < 8) scount[threadIdx.x] = 0;
+    __shared__ uint32_t lh[256], lz[256];
+    const bool sectors = rmode == RAY_SECTORS, azimuth = rmode == RAY_AZIMUTH;
+    if (sectors && threadIdx.x < 8) scount[threadIdx.x] = 0;
+    if (azimuth) lz[threadIdx.x] = 0;
     if (hist) lh[threadIdx.x] = 0;
-    if (rsec || hist) __syncthreads();
+    if (rmode || hist) __syncthreads();
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    // the block's 256 points lie in one tile (256 divides RS_TILE); azimuth counts are per tile
+    // and scan, so a block over several scans counts into global memory directly
+    const int64_t tile = ((int64_t)blockIdx.x * 256 / RS_TILE) * 256;
+    int az_scan = 0;
+    if (azimuth && S > 1 && NT > 0) {
+        const int64_t i0 = (int64_t)blockIdx.x * 256, i1 = i0 + 255 < NT ? i0 + 255 : NT - 1;
+        const int s0 = scan_of(sd, S, i0);
+        az_scan = s0 == scan_of(sd, S, i1) ? s0 : -1;
+    }
     if (i < NT) {
     int s = scan_of(sd, S, i);
     const ScanDesc &d = sd[s];
@@ -142,13 +170,19 @@ __global__ __launch_bounds__(256) void k_prepare(const P *__restrict__ in, P *__
     keys[i] = key;
     vals[i] = (uint32_t)i;
     if (hist) atomicAdd(&lh[key & 0xFFu], 1u);
-    if (rsec) {
+    if (sectors) {
         int sec = 255;
         if (ok) {
             sec = ray_sector((double)x - d.ego[0], (double)y - d.ego[1]);
             atomicAdd(&scount[sec], 1);
         }
         rsec[i] = (uint8_t)sec;
+    }
+    if (azimuth && ok) {
+        const uint32_t bin = ray_azimuth_of<P>(d, x, y) >> 8;
+        if (az_scan >= 0) atomicAdd(&lz[bin], 1u);
+        else atomicAdd(&azhist[tile + 256 * s + bin], 1u);
+        rsec[i] = (uint8_t)bin;
     }
     }
     if (hist) {
@@ -158,11 +192,10 @@ __global__ __launch_bounds__(256) void k_prepare(const P *__restrict__ in, P *__
         for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < nz; k += (int64_t)gridDim.x * blockDim.x)
             hist[(1 + k / rw) * hwords + k % rw] = 0;
     }
-    if (rsec || hist) __syncthreads();
-    if (rsec && threadIdx.x < 8 && scount[threadIdx.x]) atomicAdd(&st->sec_count[threadIdx.x], scount[threadIdx.x]);
-    // the block's 256 points lie in one sort tile (256 divides RS_TILE)
-    if (hist && lh[threadIdx.x])
-        atomicAdd(&hist[((int64_t)blockIdx.x * 256 / RS_TILE) * 256 + threadIdx.x], lh[threadIdx.x]);
+    if (rmode || hist) __syncthreads();
+    if (sectors && threadIdx.x < 8 && scount[threadIdx.x]) atomicAdd(&st->sec_count[threadIdx.x], scount[threadIdx.x]);
+    if (hist && lh[threadIdx.x]) atomicAdd(&hist[tile + threadIdx.x], lh[threadIdx.x]);
+    if (azimuth && lz[threadIdx.x]) atomicAdd(&azhist[tile + 256 * az_scan + threadIdx.x], lz[threadIdx.x]);
 }
 
 // Groups valid rays by azimuth sector: each block appends its rays of sector s, in point
@@ -539,6 +572,350 @@ __global__ __launch_bounds__(256) void k_raycast(const P *__restrict__ world,
 }
 
 // ------------------------------------------------------------------------------------
+// Azimuth-ordered cast, the default.  A block traces AZ_RAYS consecutive rays of the azimuth
+// order: a wedge of the map a few columns wide, whose counts it keeps in LDS and adds to the
+// slot table once at the end, so a voxel costs one global update per wedge instead of one per
+// run of adjacent rays, and near the sensor, where every wedge meets, a few hundred.
+//
+// All rays start at the ego.  Seen along the wedge's major axis a (x or y, whichever its rays
+// follow) a ray of slope t = db/da is in column floor(b0 + d t) at distance d, so between the
+// wedge's smallest and largest slope row d (a = ego +- d) spans W(d) columns of the minor axis
+// b; the rows' columns, z_lo .. z_lo + H - 1 each (the heights the wedge's rays reach), lie one
+// after another in the LDS counters.  A step that falls outside (a ray that leads along the
+// other axis or z, a rounded edge, rows past the counters' room) updates the slot table
+// directly: the layout decides only where a step is counted.
+//
+// Counters are 16 bits, two to a word: a ray enters a voxel at most once (its dominant
+// coordinate moves one voxel a step), so a counter holds at most AZ_RAYS.
+//
+// A step is a chain of dependent instructions, so a ray's steps are dealt to several lanes: an
+// item is up to `seg` consecutive steps of one ray, and its lane first repeats the f32
+// additions of the steps before them (three instructions a step, the same rounding).  Rays of
+// all lengths give full wavefronts that way (in ring order a ray's steps fill 45 % of the lanes
+// on the headline scan), and the longest ray no longer sets the time.  The number of a ray's
+// steps comes from one division instead of an f64 sum and comparison per step (ray_steps).
+//
+// Bound by the step arithmetic and the LDS additions: on 131,072 rays into 256 x 256 x 64 (6.6M
+// steps, event-timed alone) 36 us, of which the set-up is 6, the steps without their counts 13,
+// the LDS additions 5 and the additions to the slot table 4; one lane per ray took 61 us, four
+// row reads one after another instead of together 44.  Before, the tiled cast and its conversion
+// took 60 us there (36 + 8 with k_az_order now), 125 us on 235,877 rays into 512 x 512 x 64 (76 +
+// 13), and the sort beside it 65 us instead of 15 for its first pass, starved by the cast's
+// 2.2M global updates.
+constexpr int AZ_RAYS = 256;
+constexpr int AZ_THREADS = 512;
+constexpr int AZ_DIST = 512;      // rows of the LDS layout
+constexpr int AZ_SEGS = 16;       // most items of one ray
+constexpr int AZ_SEG = 32;        // steps per item, doubled until AZ_SEGS items hold the longest ray
+constexpr int AZ_BATCH = 4;       // steps whose layout rows are read together
+static_assert(AZ_RAYS == 256 && AZ_THREADS == 2 * AZ_RAYS && AZ_DIST == AZ_THREADS,
+              "item = ray | segment << 8; one row a thread; 16-bit counters");
+static_assert(AZ_SEG % AZ_BATCH == 0, "whole batches");
+
+// LDS counters per block: the wedges' need for a scan of n rays on this map (rows of 1 + d dt
+// columns, dt = 2 x the wedge's angle on the diagonals, of about 3/4 of the heights), at most
+// 48 KiB, so that two blocks and a sort block of the other stream fit a compute unit's 160 KiB.
+inline int64_t az_lds_counters(const Geo &g, int64_t n) {
+    const double half = g.XY / 2.0 < AZ_DIST ? g.XY / 2.0 : AZ_DIST;
+    const double dt = 2.0 * 6.2832 * AZ_RAYS / (double)(n > AZ_RAYS ? n : AZ_RAYS);
+    const double need = (half + 0.5 * half * half * dt) * g.Z * 0.75;
+    int64_t c = need < 24576.0 ? (int64_t)need : 24576;
+    c = (c + 1023) / 1024 * 1024;
+    return c < 4096 ? 4096 : c;
+}
+
+// Steps of a ray by the length rule alone (gvom.py:1209-1231): the smallest j with
+// dlen + ... + dlen (j terms, summed in f64 from 0) >= rl1, at most `most`.  The sum differs
+// from j dlen by less than j^2 2^-53 dlen, so away from the integers ceil(rl1 / dlen) is it.
+__device__ __forceinline__ int32_t ray_steps(const Ray &r, int32_t most) {
+    if (!r.alive) return 0;
+    const double q = r.rl1 / r.dlen;
+    if (q > (double)most) return most;
+    const double c = ceil(q);
+    if (c - q > 1e-6 && c - q < 1.0 - 1e-6) return (int32_t)c;
+    double sum = 0.0;
+    int32_t j = 0;
+    while (sum < r.rl1 && j < most) {
+        sum += r.dlen;
+        ++j;
+    }
+    return j;
+}
+
+// Steps along one axis until coordinate p leaves [0, size) at inc per step, not fewer than the
+// march takes but for the rounding of the result.  Each f32 addition is off by at most half an
+// ulp of the coordinate, |p + o| + size at most (o the map's origin): far from the world's
+// origin small increments are lost or grow.
+__device__ __forceinline__ float steps_inside(float p, float inc, float size, int32_t o) {
+    const float slow = fabsf(inc) - (fabsf(p + (float)o) + size) * 0x1p-24f;
+    return slow > 0.0f ? (inc > 0.0f ? size - p : p) / slow : 1e9f;
+}
+
+template <typename P>
+__global__ __launch_bounds__(AZ_THREADS) void k_raycast_az(const P *__restrict__ world,
+                                                           const ScanDesc *__restrict__ sd, int S, Geo g,
+                                                           const DevState *__restrict__ st,
+                                                           int32_t *__restrict__ tables, int maxit, int force_slot,
+                                                           const uint32_t *__restrict__ order,
+                                                           uint32_t *__restrict__ azhist, int64_t azwords, int cap) {
+    extern __shared__ uint32_t cnt[];           // cap 16-bit counters
+    __shared__ uint2 row[AZ_DIST];              // first counter; first column | columns << 16
+    __shared__ float4 rays[AZ_RAYS];            // increments and steps (negative: not in the layout)
+    __shared__ uint16_t items[AZ_RAYS * AZ_SEGS];
+    __shared__ int32_t segc[AZ_SEGS * 4 + 1];
+    __shared__ float red[4][6];
+    __shared__ int loose[4];
+    __shared__ int32_t wsum[AZ_THREADS / 64];
+    __shared__ int major;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    // the counts' last reader was k_az_order: zero for the next scan stage
+    for (int64_t k = (int64_t)blockIdx.x * AZ_THREADS + t; k < azwords; k += (int64_t)gridDim.x * AZ_THREADS)
+        azhist[k] = 0;
+    // the block's scan
+    int s = 0, first = (int)blockIdx.x;
+    for (; s < S - 1; ++s) {
+        const int nb = (int)((sd[s].count + AZ_RAYS - 1) / AZ_RAYS);
+        if (first < nb) break;
+        first -= nb;
+    }
+    first *= AZ_RAYS;
+    const int32_t n = sd[s].count > 0 ? st->ray_n[s] : 0;
+    if (first >= n) return;
+    const int buf = force_slot >= 0 ? force_slot : new_buf(st->flip, (st->next_slot + s) % g.B);
+    int32_t *table = tables + (int64_t)buf * g.V;
+    const int m = n - first < AZ_RAYS ? n - first : AZ_RAYS;   // rays of this block
+    for (int k = t; k < cap / 2; k += AZ_THREADS) cnt[k] = 0;
+    // the ego's place
+    double o[3];
+    scan_origin(sd[s], g, o);
+    const int32_t o0 = (int32_t)o[0], o1 = (int32_t)o[1], oz = (int32_t)o[2];
+    const float e0 = (float)(sd[s].ego[0] / g.xy_res), e1 = (float)(sd[s].ego[1] / g.xy_res);
+    const float pz0 = (float)(sd[s].ego[2] / g.z_res);
+    // a wavefront's lanes take every fourth ray: about one azimuth of the sensor each, so that few
+    // of its lanes are in one voxel
+    const int place = ((t & 63) << 2) | (w & 3);
+    Ray r;
+    r.inc0 = r.inc1 = r.inc2 = 0.0f;
+    int32_t steps = 0;
+    if (w < 4 && place < m) {
+        ray_init<P>(r, sd[s], g, world, (int64_t)order[sd[s].offset + first + place]);
+        steps = ray_steps(r, maxit);
+    }
+    // the wedge's major axis and direction are its middle ray's
+    if (w < 4 && place == m / 2) {
+        const bool y = !(fabsf(r.inc0) >= fabsf(r.inc1));
+        major = (y ? 1 : 0) | ((y ? r.inc1 : r.inc0) < 0.0f ? 2 : 0);
+    }
+    __syncthreads();
+    const bool swap = major & 1;
+    const float dir = (major & 2) ? -1.0f : 1.0f;
+    const float pa0 = swap ? e1 : e0, pb0 = swap ? e0 : e1;
+    const int32_t oa = swap ? o1 : o0, ob = swap ? o0 : o1;
+    const int32_t ea = floor_to_i32(pa0) - oa;
+    const float b0 = pb0 - (float)ob, z0 = pz0 - (float)oz;
+    if (w < 4) {
+        const float ia = swap ? r.inc1 : r.inc0, ib = swap ? r.inc0 : r.inc1, iz = r.inc2;
+        // rays the layout serves: along the wedge's direction, not too far to its side
+        const bool fit = steps > 0 && ia * dir > 0.0f && fabsf(ib) <= 1.25f * fabsf(ia);
+        float len = (float)steps;
+        len = fminf(len, steps_inside(pa0 - (float)oa, ia, (float)g.XY, oa));
+        len = fminf(len, steps_inside(b0, ib, (float)g.XY, ob));
+        len = fminf(len, steps_inside(z0, iz, (float)g.Z, oz));
+        len = fmaxf(len, 0.0f);
+        // a ray takes no step after it has left the map
+        steps = min(steps, (int32_t)len + 2);
+        rays[place] = make_float4(ia, ib, iz, __int_as_float(fit ? steps : -steps));
+        const float slope = ib / fabsf(ia);
+        float v[6] = {fit ? slope : 1e9f, fit ? -slope : 1e9f, fit ? fminf(z0, z0 + len * iz) : 1e9f,
+                      fit ? -fmaxf(z0, z0 + len * iz) : 1e9f, fit ? -len * fabsf(ia) : 0.0f, -(float)steps};
+        const uint64_t lo = __ballot(fit && fabsf(ia) != 1.0f);
+        for (int off = 1; off < 64; off <<= 1)
+#pragma unroll
+            for (int k = 0; k < 6; ++k) v[k] = fminf(v[k], __shfl_xor(v[k], off));
+        if (lane == 0) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) red[w][k] = v[k];
+            loose[w] = lo != 0;
+        }
+    }
+    __syncthreads();
+    float v[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) v[k] = fminf(fminf(red[0][k], red[1][k]), fminf(red[2][k], red[3][k]));
+    const bool ext = loose[0] | loose[1] | loose[2] | loose[3];
+    const float t_lo = v[0], t_hi = -v[1];
+    int zlo = v[2] < 1e8f ? floor_to_i32(v[2]) : 0, zhi = v[2] < 1e8f ? floor_to_i32(-v[3]) : -1;
+    zlo = zlo < 0 ? 0 : zlo;
+    zhi = zhi > g.Z - 1 ? g.Z - 1 : zhi;
+    const int H = zhi - zlo + 1 > 0 ? zhi - zlo + 1 : 0;
+    // the last row stays empty: steps beyond it read it and find no counter
+    const int dmax = H > 0 ? (int)fminf(-v[4] + 1.0f, (float)(AZ_DIST - 2)) : -1;
+    const int longest = (int)-v[5];
+    int seg = AZ_SEG;
+    while (seg * AZ_SEGS < longest) seg <<= 1;
+    // row t: columns, and its first counter by a scan over the block
+    int lo_col, width, size;
+    {
+        const int d = t;
+        // dominant rays are at exactly d voxels after d steps; others anywhere within the row
+        const float x0 = ext ? (float)(d - 1) : (float)d, x1 = ext ? (float)(d + 1) : (float)d;
+        int lo = floor_to_i32(b0 + fminf(x0 * t_lo, x1 * t_lo)), hi = floor_to_i32(b0 + fmaxf(x0 * t_hi, x1 * t_hi));
+        lo = lo < 0 ? 0 : lo;
+        hi = hi > g.XY - 1 ? g.XY - 1 : hi;
+        lo_col = lo;
+        const int a = dir > 0.0f ? ea + d : ea - d;
+        width = d <= dmax && hi >= lo && (uint32_t)a < (uint32_t)g.XY ? hi - lo + 1 : 0;
+        size = width * H;
+    }
+    int32_t sum = size;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int32_t u = __shfl_up(sum, off);
+        if (lane >= off) sum += u;
+    }
+    if (lane == 63) wsum[w] = sum;
+    // items: segment k of every ray longer than k seg, segment by segment
+    const int32_t mine = w < 4 ? __float_as_int(rays[t].w) : 0;
+    if (w < 4)
+        for (int k = 0; k < AZ_SEGS; ++k) {
+            const uint64_t b = __ballot(mine > k * seg);
+            if (lane == 0) segc[k * 4 + w] = __popcll(b);
+        }
+    __syncthreads();
+    int32_t at = sum - size;
+    for (int ww = 0; ww < w; ++ww) at += wsum[ww];
+    // rows past the counters' room stay empty
+    row[t] = make_uint2((uint32_t)at, (uint32_t)lo_col | (uint32_t)(at + size <= cap ? width : 0) << 16);
+    if (w == 7) {
+        const int32_t c = segc[lane];
+        int32_t p = c;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int32_t u = __shfl_up(p, off);
+            if (lane >= off) p += u;
+        }
+        segc[lane] = p - c;
+        if (lane == 63) segc[64] = p;
+    }
+    __syncthreads();
+    if (w < 4)
+        for (int k = 0; k < AZ_SEGS; ++k) {
+            const uint64_t b = __ballot(mine > k * seg);
+            if (b == 0ull) break;
+            if (mine > k * seg)
+                items[segc[k * 4 + w] + __popcll(b & ((1ull << lane) - 1ull))] = (uint16_t)(t | (k << 8));
+        }
+    __syncthreads();
+    const int32_t n_items = segc[64];
+    const uint32_t XY = (uint32_t)g.XY, Z = (uint32_t)g.Z;
+    const uint32_t sa = swap ? Z : XY * Z, sb = swap ? XY * Z : Z;
+    // d = |a - ego|: (floor(pa) ^ flip) + d0
+    const int32_t flip = dir > 0.0f ? 0 : -1, d0 = dir > 0.0f ? -(oa + ea) : oa + ea + 1;
+    const int32_t zbase = oz + zlo;
+    for (int i0 = w * 64; i0 < n_items; i0 += AZ_THREADS) {
+        const bool have = i0 + lane < n_items;
+        const uint32_t it = have ? items[i0 + lane] : 0u;
+        const float4 ry = rays[it & 255u];
+        const int32_t from = (int32_t)(it >> 8) * seg;
+        float pa = pa0, pb = pb0, pz = pz0;
+        // the additions of the steps before this item (a wavefront's items mostly share the segment)
+        for (int k = 0; __ballot(k < from); k += AZ_SEG) {
+            if (k < from)
+#pragma unroll 8
+                for (int q = 0; q < AZ_SEG; ++q) {
+                    pa += ry.x;
+                    pb += ry.y;
+                    pz += ry.z;
+                }
+        }
+        const int32_t left = have ? min(__float_as_int(ry.w) - from, seg) : 0;
+        // near the sensor many of a wavefront's rays are in one voxel: one addition per run of
+        // neighbouring lanes instead of one LDS conflict per ray
+        const bool merge = __ballot(have && from == 0) != 0ull;
+        for (int k = 0; k < seg; k += AZ_BATCH) {
+            if (__ballot(k < left) == 0ull) break;
+            int32_t fa[AZ_BATCH], fb[AZ_BATCH], fz[AZ_BATCH];
+            uint2 rw[AZ_BATCH];
+#pragma unroll
+            for (int u = 0; u < AZ_BATCH; ++u) {
+                pa += ry.x;
+                pb += ry.y;
+                pz += ry.z;
+                // floor(pt - origin) in f64 (gvom.py:1215-1223) = floor(pt) - origin, as in ray_advance
+                fa[u] = floor_to_i32(pa);
+                fb[u] = floor_to_i32(pb) - ob;
+                fz[u] = floor_to_i32(pz);
+                rw[u] = row[min((uint32_t)((fa[u] ^ flip) + d0), (uint32_t)(AZ_DIST - 1))];
+            }
+            uint64_t other = 0ull;
+            bool out[AZ_BATCH];
+#pragma unroll
+            for (int u = 0; u < AZ_BATCH; ++u) {
+                // a counter's row and column lie on the map, so a step with a counter is on it
+                const uint32_t rel = (uint32_t)fb[u] - (rw[u].y & 0xFFFFu), zr = (uint32_t)(fz[u] - zbase);
+                const bool live = k + u < left;
+                const bool here = live & (rel < (rw[u].y >> 16)) & (zr < (uint32_t)H);
+                const uint32_t q = rw[u].x + __umul24(rel, (uint32_t)H) + zr;
+                if (merge) {
+                    const uint32_t c = (uint32_t)run_length_sel(here ? q : 0xFFFFFFFFu - (uint32_t)lane, lane);
+                    if (c) atomicAdd(&cnt[q >> 1], c << ((q & 1u) << 4));
+                } else if (here) {
+                    atomicAdd(&cnt[q >> 1], 1u << ((q & 1u) << 4));
+                }
+                out[u] = live & !here;
+                other |= __ballot(out[u]);
+            }
+            if (other) {
+                // steps without a counter: off the map (where a ray takes no step), or counted in the
+                // slot table
+#pragma unroll
+                for (int u = 0; u < AZ_BATCH; ++u) {
+                    const uint32_t a = (uint32_t)(fa[u] - oa), b = (uint32_t)fb[u], z = (uint32_t)(fz[u] - oz);
+                    if (out[u] & (a < XY) & (b < XY) & (z < Z))
+                        __hip_atomic_fetch_add(table + (__umul24(a, sa) + __umul24(b, sb) + z), 1, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+        }
+    }
+    // rays the layout does not serve
+    if (w < 4 && __ballot(mine < 0)) {
+        const float4 ry = rays[t];
+        float pa = pa0, pb = pb0, pz = pz0;
+        for (int k = 0; __ballot(k < -mine); ++k) {
+            pa += ry.x;
+            pb += ry.y;
+            pz += ry.z;
+            const uint32_t a = (uint32_t)(floor_to_i32(pa) - oa), b = (uint32_t)(floor_to_i32(pb) - ob);
+            const uint32_t z = (uint32_t)(floor_to_i32(pz) - oz);
+            const uint32_t at = __umul24(a, sa) + __umul24(b, sb) + z;
+            const bool on = (k < -mine) & (a < XY) & (b < XY) & (z < Z);
+            const int c = run_length_sel(on ? at : 0xFFFFFFFFu - (uint32_t)lane, lane);
+            if (c) __hip_atomic_fetch_add(table + at, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    __syncthreads();
+    // one wavefront per row: its columns' counts to the slot table, lanes along z
+    const uint16_t *c16 = reinterpret_cast<const uint16_t *>(cnt);
+    const float inv = 1.0f / (float)(H > 0 ? H : 1);
+    for (int d = w; d <= dmax; d += AZ_THREADS / 64) {
+        const uint2 rw = row[d];
+        const uint32_t W = rw.y >> 16, lo = rw.y & 0xFFFFu;
+        const uint32_t a = (uint32_t)(dir > 0.0f ? ea + d : ea - d);
+        if (W == 0) continue;
+        const uint32_t nq = W * (uint32_t)H;
+        int32_t *base = table + a * sa + lo * sb + zlo;
+#pragma unroll 2
+        for (uint32_t q = lane; q < nq; q += 64) {
+            const int32_t c = c16[rw.x + q];
+            // q / H: q < 2^15 and the quotient's fraction is at least 1 / (2 H) away from an integer
+            const uint32_t rel = (uint32_t)(((float)q + 0.5f) * inv);
+            if (c)
+                __hip_atomic_fetch_add(base + rel * sb + (q - rel * (uint32_t)H), c, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------
 // Radix sort: 8-bit digits, tiles of RS_TILE keys (defined with k_prepare).
 // Points per moment chunk (one wavefront, see mom_chunk).
 constexpr int MCH = 64;
@@ -701,6 +1078,113 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint32_t *__res
     if (threadIdx.x < GVOM_MAX_BATCH && scn[threadIdx.x]) atomicAdd(&scan_cnt[threadIdx.x], scn[threadIdx.x]);
     __syncthreads();
     rs_scatter_tile(kout, vout, n, shift, base, lane, w, wcnt, gbase, kk, vv, lo);
+}
+
+// The azimuth order: per scan, a stable scatter of the valid rays' indices by azimuth bin, as
+// the sort's first pass (hist: bin counts per row from k_prepare), by one block per row b < nblk
+// (the points of one scan in one tile, see az_rows); the blocks after them clear the S target slot tables, RS_THREADS x 16 words each, which the cast counts into.
+constexpr int CLEAR_WORDS = RS_THREADS * 16;
+
+__global__ __launch_bounds__(RS_THREADS) void k_az_order(const uint8_t *__restrict__ rbin,
+                                                         const uint8_t *__restrict__ valid,
+                                                         const ScanDesc *__restrict__ sd, int S, int nblk,
+                                                         const uint32_t *__restrict__ hist,
+                                                         uint32_t *__restrict__ order, DevState *__restrict__ st,
+                                                         int32_t *__restrict__ tables, int B, int32_t V,
+                                                         int clear_blocks, int force_slot) {
+    __shared__ uint32_t wcnt[RS_WAVES][256];
+    __shared__ uint32_t ptot[4][256], pbef[4][256];
+    __shared__ uint32_t gbase[256];
+    __shared__ uint32_t wtot[4];
+    if ((int)blockIdx.x >= nblk) {
+        const int cb = (int)blockIdx.x - nblk, s = cb / clear_blocks;
+        const int buf =
+            force_slot >= 0 ? force_slot : __builtin_amdgcn_readfirstlane(new_buf(st->flip, (st->next_slot + s) % B));
+        int32_t *t = tables + (int64_t)buf * V;
+        const int64_t base = (int64_t)(cb - s * clear_blocks) * CLEAR_WORDS;
+        if ((V & 3) == 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int64_t j = base + (k * RS_THREADS + (int)threadIdx.x) * 4;
+                if (j < V) *reinterpret_cast<int4 *>(t + j) = make_int4(0, 0, 0, 0);
+            }
+        } else {
+            for (int k = 0; k < 16; ++k) {
+                const int64_t j = base + k * RS_THREADS + (int)threadIdx.x;
+                if (j < V) t[j] = 0;
+            }
+        }
+        return;
+    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int me = (int)blockIdx.x;
+    // the row's scan: rows [r0, r1] of scan s
+    int s = 0, r0 = 0, r1 = -1;
+    int64_t beg = 0, end = 0;
+    for (; s < S; ++s) {
+        beg = sd[s].offset;
+        end = beg + sd[s].count;
+        if (end == beg) continue;
+        r0 = (int)(beg / RS_TILE) + s;
+        r1 = (int)((end - 1) / RS_TILE) + s;
+        if (me <= r1) break;
+    }
+    if (s == S || me < r0) return;   // a row between two scans' rows (uniform)
+    for (int k = threadIdx.x; k < RS_WAVES * 256; k += RS_THREADS) (&wcnt[0][0])[k] = 0;
+    {
+        const int d = threadIdx.x & 255, q = threadIdx.x >> 8;
+        uint32_t before = 0, total = 0;
+#pragma unroll 8
+        for (int b = r0 + q; b <= r1; b += 4) {
+            const uint32_t c = hist[(int64_t)b * 256 + d];
+            total += c;
+            before += (b < me) ? c : 0u;
+        }
+        ptot[q][d] = total;
+        pbef[q][d] = before;
+    }
+    __syncthreads();
+    const uint64_t lt = (1ull << lane) - 1ull;
+    const int64_t base = (int64_t)(me - s) * RS_TILE + w * (RS_ROWS * 64);
+    uint32_t dd[RS_ROWS], lo[RS_ROWS];
+    bool in[RS_ROWS];
+#pragma unroll
+    for (int r = 0; r < RS_ROWS; ++r) {
+        const int64_t i = base + r * 64 + lane;
+        in[r] = i >= beg && i < end && valid[i];
+        dd[r] = in[r] ? rbin[i] : 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < RS_ROWS; ++r) {
+        uint64_t m = __ballot(in[r]);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const bool bit = (dd[r] >> b) & 1u;
+            const uint64_t bb = __ballot(bit);
+            m &= bit ? bb : ~bb;
+        }
+        const uint32_t rank = __popcll(m & lt), cnt = __popcll(m);
+        const uint32_t prior = wcnt[w][dd[r]];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        if (in[r] && rank == cnt - 1) wcnt[w][dd[r]] = prior + cnt;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        lo[r] = prior + rank;
+    }
+    if (threadIdx.x < 256) {
+        const int d = threadIdx.x;
+        ptot[0][d] = rs_digit_scan(ptot[0][d] + ptot[1][d] + ptot[2][d] + ptot[3][d], lane, w, wtot) +
+                     pbef[0][d] + pbef[1][d] + pbef[2][d] + pbef[3][d];
+    }
+    __syncthreads();
+    if (threadIdx.x < 256) {
+        gbase[threadIdx.x] = rs_digit_add(wtot, w) + ptot[0][threadIdx.x];
+        rs_wave_offsets(wcnt, threadIdx.x);
+    }
+    if (me == r0 && threadIdx.x == 0) st->ray_n[s] = (int32_t)rs_digit_add(wtot, 4);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RS_ROWS; ++r)
+        if (in[r]) order[beg + gbase[dd[r]] + wcnt[w][dd[r]] + lo[r]] = (uint32_t)(base + r * 64 + lane);
 }
 
 // Later passes, without a histogram kernel: each tile ranks its keys, publishes its digit
@@ -1366,14 +1850,16 @@ hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t s) {
 
 hipError_t launch_prepare(int dtype, const void *in, void *world, uint32_t *keys, uint32_t *vals,
                           uint8_t *valid, const ScanDesc *sd, int S, int64_t NT, const Geo &g,
-                          DevState *st, uint8_t *rsec, uint32_t *hist, int64_t hwords, hipStream_t s) {
+                          DevState *st, int rmode, uint8_t *rsec, uint32_t *hist, int64_t hwords, uint32_t *azhist,
+                          int64_t azwords, hipStream_t s) {
+    if (rmode == RAY_AZIMUTH && (!azhist || gvom_plan::az_hist_words(NT, S) > azwords)) return hipErrorInvalidValue;
     unsigned nb = nblocks(NT, 256);
     if (dtype == GVOM_F32)
         k_prepare<float><<<nb, 256, 0, s>>>((const float *)in, (float *)world, keys, vals, valid, sd, S, NT, g, st,
-                                             rsec, hist, hwords);
+                                             rmode, rsec, hist, hwords, azhist);
     else
         k_prepare<double><<<nb, 256, 0, s>>>((const double *)in, (double *)world, keys, vals, valid, sd, S, NT, g, st,
-                                              rsec, hist, hwords);
+                                              rmode, rsec, hist, hwords, azhist);
     return hipGetLastError();
 }
 
@@ -1415,6 +1901,38 @@ hipError_t launch_raycast(int dtype, const void *world, const uint8_t *valid, co
         else RAY_LAUNCH(double, false, false);
     }
 #undef RAY_LAUNCH
+    return hipGetLastError();
+}
+
+hipError_t launch_az_order(const uint8_t *rbin, const uint8_t *valid, const ScanDesc *sd, int S, int64_t NT,
+                           const Geo &g, DevState *st, const uint32_t *azhist, int64_t azwords, uint32_t *order,
+                           int32_t *tables, int64_t table_words, int force_slot, hipStream_t s) {
+    if (S < 1 || S > GVOM_MAX_BATCH || gvom_plan::az_hist_words(NT, S) > azwords ||
+        gvom_plan::slot_table_footprint(g.V, g.B, force_slot) > table_words)
+        return hipErrorInvalidValue;
+    const unsigned rows = (unsigned)gvom_plan::az_rows(NT, S), cb = nblocks(g.V, CLEAR_WORDS);
+    k_az_order<<<rows + cb * (unsigned)S, RS_THREADS, 0, s>>>(rbin, valid, sd, S, (int)rows, azhist, order, st, tables,
+                                                              g.B, (int32_t)g.V, (int)cb, force_slot);
+    return hipGetLastError();
+}
+
+hipError_t launch_raycast_az(int dtype, const void *world, const ScanDesc *sd, int S, int64_t NT, const Geo &g,
+                             const DevState *st, int32_t *tables, int64_t table_words, const uint32_t *order,
+                             uint32_t *azhist, int64_t azwords, int clear_counts, int force_slot, hipStream_t s) {
+    if (S < 1 || S > GVOM_MAX_BATCH || gvom_plan::slot_table_footprint(g.V, g.B, force_slot) > table_words ||
+        gvom_plan::az_hist_words(NT, S) > azwords)
+        return hipErrorInvalidValue;
+    const int maxit = (g.XY > g.Z ? g.XY : g.Z) + 2;
+    const int64_t words = clear_counts ? gvom_plan::az_hist_words(NT, S) : 0;
+    const unsigned nb = nblocks(NT, AZ_RAYS) + (unsigned)S - 1;   // >= the scans' blocks
+    const int64_t cap = az_lds_counters(g, NT / S);
+    const size_t lds = (size_t)cap * 2;
+    if (dtype == GVOM_F32)
+        k_raycast_az<float><<<nb, AZ_THREADS, lds, s>>>((const float *)world, sd, S, g, st, tables, maxit, force_slot,
+                                                     order, azhist, words, (int)cap);
+    else
+        k_raycast_az<double><<<nb, AZ_THREADS, lds, s>>>((const double *)world, sd, S, g, st, tables, maxit, force_slot,
+                                                      order, azhist, words, (int)cap);
     return hipGetLastError();
 }
 

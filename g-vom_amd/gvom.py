@@ -197,7 +197,7 @@ class Gvom:
     def autotune(self, dev_points, n, ego_position, transform=None, dtype=np.float32):
         """Pick the ray-cast variant by timing it on one device-resident scan.  Returns
         (block, rays_per_thread, flags, best_ms); flags bit 0 LDS box, bit 1 sector order,
-        bit 2 tiled scratch, bit 3 spread (kept as set, not searched)."""
+        bit 2 tiled scratch, bit 3 spread (kept as set, not searched), bit 4 azimuth order."""
         ptr = dev_points.ptr if isinstance(dev_points, nat.DeviceArray) else ctypes.c_void_p(int(dev_points))
         ego = np.ascontiguousarray(np.asarray(ego_position, dtype=np.float64).reshape(3))
         T, tdt = _as_transform(transform)
@@ -218,10 +218,12 @@ class Gvom:
         return out[0], int(out[1])
 
     def set_raycast_config(self, block=128, rays_per_thread=1, use_box=False, sector_order=False, tiled=True,
-                           spread=True):
+                           spread=True, azimuth=False):
         """Ray-cast launch shape and variant (tiled scratch excludes the LDS box; spread takes
-        each block's wavefronts from across the scan); a new handle starts at the defaults."""
-        flags = (1 if use_box else 0) | (2 if sector_order else 0) | (4 if tiled else 0) | (8 if spread else 0)
+        each block's wavefronts from across the scan).  azimuth=True, as a new handle starts: scans
+        of at least 12e6 points x xy_size are cast in azimuth order, smaller ones as set here."""
+        flags = ((1 if use_box else 0) | (2 if sector_order else 0) | (4 if tiled else 0) | (8 if spread else 0) |
+                 (16 if azimuth else 0))
         nat.check(self._lib.gvom_set_raycast_config(self._h, int(block), int(rays_per_thread), flags), self._h)
 
     def set_ray_rings(self, points_per_ring, patch_rings=32):
