@@ -287,7 +287,8 @@ static hipError_t join_metrics(gvom_handle *h) {
 }
 
 static void free_all(gvom_handle *h) {
-    void *ptrs[] = {h->st, h->slot_tables, h->slot_recs, h->comb_tables, h->comb_recs, h->height, h->inferred,
+    void *ptrs[] = {h->st, h->slot_tables ? h->slot_tables - TABLE_PAD : nullptr, h->slot_recs,
+                    h->comb_tables ? h->comb_tables - TABLE_PAD : nullptr, h->comb_recs, h->height, h->inferred,
                     h->slope_x, h->slope_y, h->maps_block, h->delta, h->occ_list,
                     h->col_count, h->chunk_tot, h->export_buf, h->pts_in, h->world, h->valid, h->k0, h->v0, h->k1, h->v1,
                     h->hist, h->blk, h->seg_key, h->seg_start, h->mom, h->part, h->sd, h->diff_rec,
@@ -411,9 +412,11 @@ extern "C" int gvom_create(const gvom_params *params, gvom_handle **out) {
     CKC(dalloc(&h->st, 1));
     CKC(hipMemset(h->st, 0, sizeof(DevState)));
     h->slot_table_words = gvom_plan::alloc_slot_table_words(V, g.B);   // two buffers per ring slot
-    CKC(dalloc(&h->slot_tables, h->slot_table_words));
+    CKC(dalloc(&h->slot_tables, h->slot_table_words + 2 * TABLE_PAD));
+    h->slot_tables += TABLE_PAD;
     h->ccap = V;
-    CKC(dalloc(&h->comb_tables, 2 * V));
+    CKC(dalloc(&h->comb_tables, 2 * V + 2 * TABLE_PAD));
+    h->comb_tables += TABLE_PAD;
     CKC(dalloc(&h->comb_recs, 2 * h->ccap));
     const int64_t X = g.X;
     CKC(dalloc(&h->height, X));

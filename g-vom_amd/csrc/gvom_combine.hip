@@ -2,8 +2,8 @@
 // scripts/gvom.py:222-393).
 //
 // Launch sequence (stream-ordered, no host synchronisation):
-//   tables    one wavefront per z-contiguous column: for each voxel, union of the
-//             filled slots' occupancy (slot order) and sum of their free passes, then
+//   tables    eight voxels of a z-contiguous column per lane: for each voxel, union of
+//             the filled slots' occupancy (slot order) and sum of their free passes, then
 //             the previous combined map with its <= 10-pass carry-over rule
 //             (gvom.py:1010-1063).  Writes OCC | source-mask or the pass count, and
 //             the column's occupied count.
@@ -52,16 +52,38 @@ __device__ __forceinline__ SrcCol source_column(const int32_t *table, const doub
 }
 
 // ------------------------------------------------------------------------------------
-// One wavefront handles CPW consecutive columns (lane = z).  The shifted source columns
-// of all sources of a group are computed from uniform data first; then every lane
-// issues its CPW x group loads before it uses the first value, so a wavefront keeps
-// CPW * (group + 1) independent loads in flight.
-constexpr int CPW = 4;
-constexpr int SRC_GROUP = 8;
+// Table pass.  A wavefront combines cpw consecutive columns, zl lanes per column, eight
+// consecutive voxels per lane (zl = ceil(z_size / 8), cpw = 64 / zl: 8 columns at z_size 64).
+// A source is the lane's own index plus one uniform offset, so its eight words come from two
+// 16-byte loads (4-byte aligned: the offset is any number of voxels) and one address; lanes
+// whose column or heights are off the source's map read a page of zeros, and where the shift
+// in z leaves a column's ends partly off the map the words are masked.  Per word and source
+// the arithmetic is one funnel shift (the sign bits collect the source mask) and a max-add.
+//
+// Bound by the reads: 256 x 256 x 64 with 8 slots (168 MB) takes 27.1 us, 6.2 TB/s, where a large
+// copy reaches 5.2 and one that stays in the Infinity Cache 8.4; 512 x 512 x 64 (671 MB) 129 us.
+// Before, a lane per voxel with four-byte loads issued about 16 vector instructions per word,
+// most of them to form and select its address: 29.3 and 133 us, and 40.0 us for 250 x 250 x 60
+// with 4 slots and 31.9 for 151 x 151 x 100 with 3 (18.4 and 13.1 now), whose sides, no multiple
+// of 8, took a slower kernel.
+constexpr int ZPL = 8;           // voxels per lane
+constexpr int SRC_GROUP = 4;     // sources loaded together
+constexpr int ZERO_PAGE_WORDS = 64;
+static_assert(ZPL == 8, "two 16-byte loads, one byte of occupancy bits per lane");
 
-__device__ __forceinline__ void col_xy(int64_t c, const Geo &g, int64_t &x, int64_t &y) {
-    x = c / g.XY;
-    y = c - x * g.XY;
+// four words at a 4-byte aligned address
+typedef int32_t words4 __attribute__((ext_vector_type(4), aligned(4)));
+
+struct Words8 {
+    words4 a, b;
+    __device__ __forceinline__ int32_t get(int j) const { return j < 4 ? a[j] : b[j - 4]; }
+};
+
+__device__ __forceinline__ Words8 load8(const int32_t *p) {
+    Words8 w;
+    w.a = *reinterpret_cast<const words4 *>(p);
+    w.b = *reinterpret_cast<const words4 *>(p + 4);
+    return w;
 }
 
 // Wave-uniform int32 in a scalar register.
@@ -69,304 +91,140 @@ __device__ __forceinline__ int32_t uni(int32_t v) { return __builtin_amdgcn_read
 
 __global__ __launch_bounds__(256) void k_comb_tables(Geo g, const DevState *__restrict__ st,
                                                      const int32_t *__restrict__ slot_tables,
+                                                     const int32_t *__restrict__ zero_page,
                                                      int32_t *__restrict__ comb_tables,
                                                      int32_t *__restrict__ col_count,
-                                                     uint64_t *__restrict__ occ_bits,
-                                                     double *__restrict__ height,
-                                                     double *__restrict__ inferred) {
-    // Everything but the z index is uniform across the wavefront: column coordinates,
-    // each source's shift and column base live in scalar registers, so a source word costs
-    // one vector compare and one load (SGPR base + lane offset).  All offsets fit in 32 bits
-    // (V * (B + 1) < 2^31).
-    const int lane = threadIdx.x & 63;
-    const int32_t XY = g.XY, Z = g.Z, X = (int32_t)g.X, V = (int32_t)g.V;
-    const int32_t c0 = uni((int32_t)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * CPW);
-    if (c0 >= X) return;
-    const int parity = uni(st->parity), cur = 1 - parity;
-    const int filled = uni(st->filled_mask), have_last = uni(st->have_last);
-    const int last_slot = uni(st->last_slot), flip = uni(st->flip);
-    const double *co = st->slot_origin[last_slot];   // combined origin = newest slot's (gvom.py:229)
-    int32_t cx[CPW], cy[CPW];
-    {
-        const int32_t x0 = uni(c0 / XY), y0 = uni(c0 - (c0 / XY) * XY);
-        int32_t x = x0, y = y0;
-#pragma unroll
-        for (int j = 0; j < CPW; ++j) {
-            cx[j] = x;
-            cy[j] = y;
-            if (++y == XY) { y = 0; ++x; }
-        }
-    }
-    const int32_t *ltab = comb_tables + (int64_t)parity * V;
-    uint32_t count[CPW] = {0, 0, 0, 0};
-    int first_free[CPW] = {-1, -1, -1, -1};
+                                                     uint64_t *__restrict__ occ_bits, double *__restrict__ height,
+                                                     double *__restrict__ inferred, int zl, int cpw) {
+    // per wavefront: a byte of occupied and a byte of free bits (passes, no hit) per lane, as
+    // 64-bit words of its columns
+    __shared__ __align__(16) uint8_t occ_b[4][512], free_b[4][512];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int32_t XY = g.XY, Z = g.Z, X = (int32_t)g.X;
     const int NW = (Z + 63) >> 6;   // occupancy words per column
-    for (int z0 = 0; z0 < Z; z0 += 64) {
-        const int z = z0 + lane;
-        const bool zin = z < Z;
-        // previous combined map
-        int32_t vl[CPW];
-        bool okl[CPW];
-        {
-            const int32_t dx = have_last ? uni((int32_t)(co[0] - st->comb_origin[parity][0])) : 0;
-            const int32_t dy = have_last ? uni((int32_t)(co[1] - st->comb_origin[parity][1])) : 0;
-            const int32_t dz = have_last ? uni((int32_t)(co[2] - st->comb_origin[parity][2])) : 0;
-            const int zl = z + dz;
-            const bool zok = have_last && zin && zl >= 0 && zl < Z;
-#pragma unroll
-            for (int j = 0; j < CPW; ++j) {
-                const int32_t ux = cx[j] + dx, uy = cy[j] + dy;
-                const bool cok = c0 + j < X && ux >= 0 && ux < XY && uy >= 0 && uy < XY;   // uniform
-                const int32_t *col = ltab + uni(cok ? (ux * XY + uy) * Z : 0);
-                okl[j] = cok && zok;
-                vl[j] = okl[j] ? col[zl] : 0;
-            }
-        }
-        uint32_t mask[CPW] = {0, 0, 0, 0}, P[CPW] = {0, 0, 0, 0};
-        for (int s0 = 0; s0 < g.B; s0 += SRC_GROUP) {
-            int32_t v[SRC_GROUP][CPW];
-#pragma unroll
-            for (int k = 0; k < SRC_GROUP; ++k) {
-                const int s = s0 + k;
-                const bool use = s < g.B && ((filled >> s) & 1);
-                const double *so = st->slot_origin[use ? s : 0];
-                const int32_t dx = uni((int32_t)(co[0] - so[0])), dy = uni((int32_t)(co[1] - so[1]));
-                const int32_t dz = uni((int32_t)(co[2] - so[2]));
-                const int zs = z + dz;
-                const bool zok = use && zin && zs >= 0 && zs < Z;
-                const int32_t *tab = slot_tables + (int64_t)cur_buf(flip, use ? s : 0) * V;
-#pragma unroll
-                for (int j = 0; j < CPW; ++j) {
-                    const int32_t ux = cx[j] + dx, uy = cy[j] + dy;
-                    const bool cok = c0 + j < X && ux >= 0 && ux < XY && uy >= 0 && uy < XY;   // uniform
-                    const int32_t *col = tab + uni(cok ? (ux * XY + uy) * Z : 0);
-                    // unused sources and off-map cells read as "no data" (0)
-                    v[k][j] = (cok && zok) ? col[zs] : 0;
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < SRC_GROUP; ++k)
-#pragma unroll
-                for (int j = 0; j < CPW; ++j) {
-                    if (v[k][j] < 0) mask[j] |= 1u << (s0 + k);
-                    else P[j] += (uint32_t)v[k][j];
-                }
-        }
-        int32_t *out = comb_tables + (int64_t)cur * V + c0 * Z;
-#pragma unroll
-        for (int j = 0; j < CPW; ++j) {
-            uint32_t m = mask[j], p = P[j];
-            if (okl[j]) {
-                if (m) {
-                    if (vl[j] < 0) m |= 1u << LAST_BIT;
-                } else if (vl[j] < 0) {
-                    if (p <= 10u) m = 1u << LAST_BIT;   // carry-over (gvom.py:1058)
-                } else {
-                    p += (uint32_t)vl[j];
-                }
-            }
-            const int32_t o = m ? (int32_t)(GVOM_OCC | m) : (int32_t)p;
-            if (zin && c0 + j < X) out[j * Z + z] = o;
-            const uint64_t ob = __ballot(m != 0);
-            count[j] += __popcll(ob);
-            if (lane == 0 && c0 + j < X) occ_bits[(int64_t)(c0 + j) * NW + (z0 >> 6)] = ob;
-            // lowest free voxel with at least one pass (gvom.py:580-590)
-            const uint64_t fb = __ballot(zin && m == 0 && p >= 1u);
-            if (first_free[j] < 0 && fb) first_free[j] = z0 + __builtin_ctzll(fb);
-        }
-    }
-    if (lane < CPW && c0 + lane < X) {
-        uint32_t cnt = count[0];
-        int ff = first_free[0];
-#pragma unroll
-        for (int j = 1; j < CPW; ++j)
-            if (lane == j) {
-                cnt = count[j];
-                ff = first_free[j];
-            }
-        const int32_t c = c0 + lane;
-        col_count[c] = (int32_t)cnt;
-        inferred[c] = ff >= 0 ? ((double)ff + co[2]) * g.z_res : -1000.0;
-        if (cnt == 0) {
-            // no occupied voxel: the robot-radius default around the latest ego, measured to
-            // the cell corner (gvom.py:561-570), else unknown (-1000); occupied columns get
-            // their height from the record merge
-            const int32_t x = c / XY, y = c - (c / XY) * XY;
-            const double *ego = st->latest_ego;
-            double h = -1000.0;
-            const double xp = ((co[0] + (double)x) * g.xy_res) - ego[0];
-            const double yp = ((co[1] + (double)y) * g.xy_res) - ego[1];
-            if (xp * xp + yp * yp <= g.robot_r * g.robot_r) h = ego[2] - g.g2l;
-            height[c] = h;
-        }
-    }
-}
-
-// Same combine for xy_size % 8 == 0, with less scalar work per column.  The RCPW columns of
-// a group lie in one x row; each source's shift (precomputed by the scan stage's commit) gives
-// one uniform column pointer, and a word that is off the map (column or z) is read from a
-// zero page instead of being masked after the load, so no per-word predicate outlives its
-// address.  A source's shift and column base are scalar work done once per group, so a wider
-// group spends less of it per column: on 256 x 256 x 64 with 8 slots, 4 columns per wavefront
-// took 29.4 us, 8 columns with 4 sources loaded together 28.6 us (8 sources together: 129
-// VGPRs, 3 wavefronts per SIMD; 16 columns spill ~190 SGPRs).  Each wavefront handles GPW
-// groups.  (The general kernel above issues ~1200 scalar instructions per wavefront for 4
-// columns, which made it scalar-issue bound.)
-constexpr int RCPW = 8;
-constexpr int RSRC_GROUP = 4;
-constexpr int RCPW_MAX = 8;
-constexpr int GPW = 1;   // measured with 4 columns: 1 group per wavefront 34.4 us, 2 groups 35.3 us, 4 groups 36.8 us
-constexpr int ZERO_PAGE_WORDS = RCPW_MAX * 256 + 64;   // covers lane + j * z_size for z_size <= 256
-
-// combine rule of one voxel: union of the sources' occupancy and sum of their passes, then
-// the previous map (gvom.py:1010-1063)
-__device__ __forceinline__ int32_t comb_word(uint32_t m, uint32_t p, bool okl, int32_t vl, bool &occ, bool &freev) {
-    if (okl) {
-        if (m) {
-            if (vl < 0) m |= 1u << LAST_BIT;
-        } else if (vl < 0) {
-            if (p <= 10u) m = 1u << LAST_BIT;   // carry-over (gvom.py:1058)
-        } else {
-            p += (uint32_t)vl;
-        }
-    }
-    occ = m != 0;
-    freev = m == 0 && p >= 1u;
-    return m ? (int32_t)(GVOM_OCC | m) : (int32_t)p;
-}
-
-__global__ __launch_bounds__(256) void k_comb_rows(Geo g, const DevState *__restrict__ st,
-                                                   const int32_t *__restrict__ slot_tables,
-                                                   const int32_t *__restrict__ zero_page,
-                                                   int32_t *__restrict__ comb_tables,
-                                                   int32_t *__restrict__ col_count,
-                                                   uint64_t *__restrict__ occ_bits,
-                                                   double *__restrict__ height,
-                                                   double *__restrict__ inferred) {
-    const int lane = threadIdx.x & 63;
-    const int32_t XY = g.XY, Z = g.Z, X = (int32_t)g.X, V = (int32_t)g.V;
-    const int32_t cw = uni((int32_t)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * (RCPW * GPW));
-    if (cw >= X) return;
+    const int32_t c0 = uni((int32_t)(blockIdx.x * 4 + wv) * cpw);
+    reinterpret_cast<uint64_t *>(occ_b[wv])[lane] = 0ull;
+    reinterpret_cast<uint64_t *>(free_b[wv])[lane] = 0ull;
+    const int cl = lane / zl, zo = lane - cl * zl, z0 = zo * ZPL;
+    const int32_t c = c0 + cl;
+    const bool act = cl < cpw && c < X;
+    const int32_t x = c / XY, y = c - x * XY;
+    const uint32_t lin = (uint32_t)c * (uint32_t)Z + (uint32_t)z0;   // V < 2^31
     const int parity = uni(st->parity), cur = 1 - parity;
     const int have_last = uni(st->have_last);
     const int last_slot = uni(st->last_slot), flip = uni(st->flip);
     const double *co = st->slot_origin[last_slot];   // combined origin = newest slot's (gvom.py:229)
-    const int32_t ldx = have_last ? uni((int32_t)(co[0] - st->comb_origin[parity][0])) : 0;
-    const int32_t ldy = have_last ? uni((int32_t)(co[1] - st->comb_origin[parity][1])) : 0;
-    const int32_t ldz = have_last ? uni((int32_t)(co[2] - st->comb_origin[parity][2])) : 0;
-    const int32_t *ltab = comb_tables + (int64_t)parity * V;
-    const int32_t *zp = zero_page + lane;
-    const int NW = (Z + 63) >> 6;
-    uint32_t count[GPW][RCPW], ffree[GPW][RCPW];
+
+    uint32_t M[ZPL], P[ZPL];
 #pragma unroll
-    for (int q = 0; q < GPW; ++q)
+    for (int j = 0; j < ZPL; ++j) M[j] = P[j] = 0;
+    // the lane's words of one source, shifted by (dx, dy, dz); reads may run up to seven words
+    // past a column's ends (the tables are padded by 64 words on both sides)
+    auto source = [&](const int32_t *tab, int32_t dx, int32_t dy, int32_t dz, bool use) {
+        const bool ok = act & use & ((uint32_t)(x + dx) < (uint32_t)XY) & ((uint32_t)(y + dy) < (uint32_t)XY) &
+                        ((uint32_t)(z0 + dz + ZPL - 1) < (uint32_t)(Z + ZPL - 1));
+        const uint32_t shift = ((uint32_t)dx * (uint32_t)XY + (uint32_t)dy) * (uint32_t)Z + (uint32_t)dz;
+        return load8(ok ? tab - ZPL + (lin + shift + ZPL) : zero_page);
+    };
+    for (int s0 = 0; s0 < g.B; s0 += SRC_GROUP) {
+        Words8 v[SRC_GROUP];
+        int32_t dz[SRC_GROUP];
 #pragma unroll
-        for (int j = 0; j < RCPW; ++j) {
-            count[q][j] = 0;
-            ffree[q][j] = 0xFFFFFFFFu;
+        for (int k = 0; k < SRC_GROUP; ++k) {
+            // shifts precomputed by the scan stage's commit (one 16-byte scalar load)
+            const int s = s0 + k < g.B ? s0 + k : 0;
+            const int4 sh = *reinterpret_cast<const int4 *>(st->comb_shift[s]);
+            dz[k] = sh.z;
+            v[k] = source(slot_tables + (int64_t)cur_buf(flip, s) * g.V, sh.x, sh.y, sh.z,
+                          (s0 + k < g.B) & (sh.w != 0));
         }
-    for (int z0 = 0; z0 < Z; z0 += 64) {
-        const int z = z0 + lane;
-        const bool zin = z < Z;
-        uint32_t mask[GPW][RCPW], P[GPW][RCPW];
 #pragma unroll
-        for (int q = 0; q < GPW; ++q)
+        for (int k = 0; k < SRC_GROUP; ++k) {
+            if (dz[k] == 0 && (Z & (ZPL - 1)) == 0) {   // uniform: every word is on the map
 #pragma unroll
-            for (int j = 0; j < RCPW; ++j) mask[q][j] = P[q][j] = 0;
-        for (int s0 = 0; s0 < g.B; s0 += RSRC_GROUP) {
-#pragma unroll
-            for (int q = 0; q < GPW; ++q) {
-                const int32_t c0 = cw + q * RCPW;
-                const int32_t x0 = c0 / XY, y0 = c0 - (c0 / XY) * XY;
-                int32_t v[RSRC_GROUP][RCPW];
-#pragma unroll
-                for (int k = 0; k < RSRC_GROUP; ++k) {
-                    // shifts precomputed by the scan stage's commit (one 16-byte scalar load)
-                    const int s = s0 + k < g.B ? s0 + k : 0;
-                    const int4 sh = *reinterpret_cast<const int4 *>(st->comb_shift[s]);
-                    const bool use = (s0 + k < g.B) & (sh.w != 0) & (c0 < X);
-                    const int32_t ux = x0 + sh.x, uy0 = y0 + sh.y;
-                    const bool rowok = use & ((uint32_t)ux < (uint32_t)XY);   // uniform
-                    const int zs = z + sh.z;
-                    const bool zok = zin & ((uint32_t)zs < (uint32_t)Z);
-                    // column j of the source: cp + j * Z (wrapping arithmetic; dereferenced
-                    // only where the column is on the map)
-                    const int32_t *cp = slot_tables + (int64_t)cur_buf(flip, s) * V +
-                                        (int32_t)(((uint32_t)ux * (uint32_t)XY + (uint32_t)uy0) * (uint32_t)Z);
-#pragma unroll
-                    for (int j = 0; j < RCPW; ++j) {
-                        const bool cok = rowok & ((uint32_t)(uy0 + j) < (uint32_t)XY);   // uniform
-                        const int32_t *a = (cok & zok) ? cp + j * Z + zs : zp + j * Z;
-                        v[k][j] = *a;
-                    }
+                for (int j = 0; j < ZPL; ++j) {
+                    const int32_t t = v[k].get(j);
+                    M[j] = __builtin_amdgcn_alignbit(M[j], (uint32_t)t, 31);   // M << 1 | sign
+                    P[j] += (uint32_t)(t > 0 ? t : 0);
                 }
+            } else {
 #pragma unroll
-                for (int k = 0; k < RSRC_GROUP; ++k)
-#pragma unroll
-                    for (int j = 0; j < RCPW; ++j) {
-                        if (v[k][j] < 0) mask[q][j] |= 1u << (s0 + k);
-                        else P[q][j] += (uint32_t)v[k][j];
-                    }
-            }
-        }
-        const int zl = z + ldz;
-        const bool zokl = (have_last != 0) & zin & ((uint32_t)zl < (uint32_t)Z);
-#pragma unroll
-        for (int q = 0; q < GPW; ++q) {
-            const int32_t c0 = cw + q * RCPW;
-            if (c0 >= X) break;
-            const int32_t x0 = c0 / XY, y0 = c0 - (c0 / XY) * XY;
-            const int32_t ux = x0 + ldx, uy0 = y0 + ldy;
-            const bool rowok = (uint32_t)ux < (uint32_t)XY;
-            const int32_t *cp = ltab + (int32_t)(((uint32_t)ux * (uint32_t)XY + (uint32_t)uy0) * (uint32_t)Z);
-            int32_t vl[RCPW];
-            bool okl[RCPW];
-#pragma unroll
-            for (int j = 0; j < RCPW; ++j) {
-                okl[j] = rowok & zokl & ((uint32_t)(uy0 + j) < (uint32_t)XY);
-                vl[j] = *(okl[j] ? cp + j * Z + zl : zp + j * Z);
-            }
-            int32_t *out = comb_tables + (int64_t)cur * V + (int64_t)c0 * Z;
-#pragma unroll
-            for (int j = 0; j < RCPW; ++j) {
-                bool occ, freev;
-                const int32_t o = comb_word(mask[q][j], P[q][j], okl[j], vl[j], occ, freev);
-                if (zin) out[j * Z + z] = o;
-                const uint64_t ob = __ballot(occ);
-                count[q][j] += __popcll(ob);
-                if (lane == 0) occ_bits[(int64_t)(c0 + j) * NW + (z0 >> 6)] = ob;
-                // lowest free voxel with at least one pass (gvom.py:580-590)
-                const uint64_t fb = __ballot(zin && freev);
-                if (ffree[q][j] == 0xFFFFFFFFu && fb) ffree[q][j] = (uint32_t)(z0 + __builtin_ctzll(fb));
+                for (int j = 0; j < ZPL; ++j) {
+                    const int32_t t = (uint32_t)(z0 + j + dz[k]) < (uint32_t)Z ? v[k].get(j) : 0;
+                    M[j] = __builtin_amdgcn_alignbit(M[j], (uint32_t)t, 31);
+                    P[j] += (uint32_t)(t > 0 ? t : 0);
+                }
             }
         }
     }
-    if (lane < GPW * RCPW) {
-        const int32_t c = cw + lane;
-        if (c < X) {
-            uint32_t cnt = 0, ff = 0xFFFFFFFFu;
+    // previous combined map
+    const int32_t ldx = have_last ? uni((int32_t)(co[0] - st->comb_origin[parity][0])) : 0;
+    const int32_t ldy = have_last ? uni((int32_t)(co[1] - st->comb_origin[parity][1])) : 0;
+    const int32_t ldz = have_last ? uni((int32_t)(co[2] - st->comb_origin[parity][2])) : 0;
+    const Words8 last = source(comb_tables + (int64_t)parity * g.V, ldx, ldy, ldz, have_last != 0);
+    const int mshift = 32 - (g.B + SRC_GROUP - 1) / SRC_GROUP * SRC_GROUP;
+    Words8 out;
+    uint32_t ob = 0, fb = 0;
 #pragma unroll
-            for (int q = 0; q < GPW; ++q)
+    for (int j = ZPL - 1; j >= 0; --j) {
+        // union of the sources' occupancy and sum of their passes, then the previous map
+        // (gvom.py:1010-1063); bit s of m: source s
+        uint32_t m = __brev(M[j]) >> mshift, p = P[j];
+        const int32_t t = (uint32_t)(z0 + j + ldz) < (uint32_t)Z ? last.get(j) : 0;
+        if (t < 0) {
+            if (m != 0 || p <= 10u) m |= 1u << LAST_BIT;   // carry-over (gvom.py:1058)
+        } else if (m == 0) {
+            p += (uint32_t)t;
+        }
+        int32_t o = m ? (int32_t)(GVOM_OCC | m) : (int32_t)p;
+        if (j < 4) out.a[j] = o;
+        else out.b[j - 4] = o;
+        o = z0 + j < Z ? o : 0;
+        ob = __builtin_amdgcn_alignbit(ob, (uint32_t)o, 31);
+        fb = __builtin_amdgcn_alignbit(fb, 0u - (uint32_t)o, 31);   // o > 0: passes
+    }
+    if (act) {
+        int32_t *dst = comb_tables + (int64_t)cur * g.V + lin;
+        if (z0 + ZPL <= Z) {
+            *reinterpret_cast<words4 *>(dst) = out.a;
+            *reinterpret_cast<words4 *>(dst + 4) = out.b;
+        } else {
 #pragma unroll
-                for (int j = 0; j < RCPW; ++j)
-                    if (lane == q * RCPW + j) {
-                        cnt = count[q][j];
-                        ff = ffree[q][j];
-                    }
-            col_count[c] = (int32_t)cnt;
-            inferred[c] = ff != 0xFFFFFFFFu ? ((double)ff + co[2]) * g.z_res : -1000.0;
-            if (cnt == 0) {
-                // no occupied voxel: the robot-radius default around the latest ego, measured to
-                // the cell corner (gvom.py:561-570), else unknown (-1000); occupied columns get
-                // their height from the record merge
-                const int32_t x = c / XY, y = c - (c / XY) * XY;
-                const double *ego = st->latest_ego;
-                double h = -1000.0;
-                const double xp = ((co[0] + (double)x) * g.xy_res) - ego[0];
-                const double yp = ((co[1] + (double)y) * g.xy_res) - ego[1];
-                if (xp * xp + yp * yp <= g.robot_r * g.robot_r) h = ego[2] - g.g2l;
-                height[c] = h;
-            }
+            for (int j = 0; j < ZPL; ++j)
+                if (z0 + j < Z) dst[j] = out.get(j);
+        }
+    }
+    __syncthreads();   // the zeroed bytes
+    if (act) {
+        occ_b[wv][cl * (8 * NW) + zo] = (uint8_t)ob;
+        free_b[wv][cl * (8 * NW) + zo] = (uint8_t)fb;
+    }
+    __syncthreads();
+    // one lane per column
+    const int32_t cc = c0 + lane;
+    if (lane < cpw && cc < X) {
+        uint32_t cnt = 0;
+        int ff = -1;
+        for (int w = 0; w < NW; ++w) {
+            const uint64_t o = reinterpret_cast<const uint64_t *>(occ_b[wv])[lane * NW + w];
+            const uint64_t f = reinterpret_cast<const uint64_t *>(free_b[wv])[lane * NW + w];
+            occ_bits[(int64_t)cc * NW + w] = o;
+            cnt += __popcll(o);
+            if (ff < 0 && f) ff = w * 64 + __builtin_ctzll(f);   // lowest free voxel (gvom.py:580-590)
+        }
+        col_count[cc] = (int32_t)cnt;
+        inferred[cc] = ff >= 0 ? ((double)ff + co[2]) * g.z_res : -1000.0;
+        if (cnt == 0) {
+            // no occupied voxel: the robot-radius default around the latest ego, measured to
+            // the cell corner (gvom.py:561-570), else unknown (-1000); occupied columns get
+            // their height from the record merge
+            const int32_t xx = cc / XY, yy = cc - xx * XY;
+            const double *ego = st->latest_ego;
+            double h = -1000.0;
+            const double xp = ((co[0] + (double)xx) * g.xy_res) - ego[0];
+            const double yp = ((co[1] + (double)yy) * g.xy_res) - ego[1];
+            if (xp * xp + yp * yp <= g.robot_r * g.robot_r) h = ego[2] - g.g2l;
+            height[cc] = h;
         }
     }
 }
@@ -959,14 +817,9 @@ int64_t zero_page_words() { return ZERO_PAGE_WORDS; }
 hipError_t launch_comb_tables(const Geo &g, DevState *st, const int32_t *slot_tables, const int32_t *zero_page,
                               int32_t *comb_tables, int32_t *col_count, uint64_t *occ_bits, double *height,
                               double *inferred, hipStream_t s) {
-    static_assert(RCPW <= RCPW_MAX, "the zero page covers RCPW_MAX columns");
-    if (g.XY % RCPW == 0 && zero_page)
-        k_comb_rows<<<nblocks((g.X + RCPW * GPW - 1) / (RCPW * GPW), 4), 256, 0, s>>>(g, st, slot_tables, zero_page,
-                                                                                 comb_tables, col_count, occ_bits,
-                                                                                 height, inferred);
-    else
-        k_comb_tables<<<nblocks((g.X + CPW - 1) / CPW, 4), 256, 0, s>>>(g, st, slot_tables, comb_tables, col_count,
-                                                                        occ_bits, height, inferred);
+    const int zl = (g.Z + ZPL - 1) / ZPL, cpw = 64 / zl;
+    k_comb_tables<<<nblocks(g.X, 4 * cpw), 256, 0, s>>>(g, st, slot_tables, zero_page, comb_tables, col_count, occ_bits,
+                                                        height, inferred, zl, cpw);
     return hipGetLastError();
 }
 

@@ -83,8 +83,9 @@ hipError_t launch_commit_process(DevState *st, const ScanDesc *sd, const Geo &g,
 // ---- combine stage (gvom_combine.hip) ----------------------------------------------------
 // Per column it also writes the occupied-voxel count, the occupancy words (bit z of word
 // z / 64), the inferred height and, for columns without occupancy, the height.
-// zero_page: zero_page_words() zeroed int32 the row kernel reads instead of off-map words
-// (xy_size % 4 == 0; null selects the general kernel).
+// zero_page: zero_page_words() zeroed int32 read instead of off-map words.  slot_tables and
+// comb_tables must be readable for TABLE_PAD words before and after.
+constexpr int64_t TABLE_PAD = 64;
 int64_t zero_page_words();
 hipError_t launch_comb_tables(const Geo &g, DevState *st, const int32_t *slot_tables, const int32_t *zero_page,
                               int32_t *comb_tables, int32_t *col_count, uint64_t *occ_bits, double *height,
