@@ -142,7 +142,8 @@ struct gvom_handle {
     void *pin_maps = nullptr, *pin_maps_dev = nullptr;   // host address and its device mapping
     uint64_t *occ_bits = nullptr;   // combined map: per column, bit z of word z / 64 = occupied
     int32_t *zero_page = nullptr;   // zeros the combine reads in place of off-map words
-    uint2 *occ_list = nullptr;
+    uint2 *occ_list = nullptr;        // compact cell list (large maps only)
+    int32_t *group_count = nullptr;   // occupied voxels per group of columns of the combined map
     int32_t *export_buf = nullptr;
     int32_t *chunk_tot = nullptr;
 
@@ -289,7 +290,7 @@ static hipError_t join_metrics(gvom_handle *h) {
 static void free_all(gvom_handle *h) {
     void *ptrs[] = {h->st, h->slot_tables ? h->slot_tables - TABLE_PAD : nullptr, h->slot_recs,
                     h->comb_tables ? h->comb_tables - TABLE_PAD : nullptr, h->comb_recs, h->height, h->inferred,
-                    h->slope_x, h->slope_y, h->maps_block, h->delta, h->occ_list,
+                    h->slope_x, h->slope_y, h->maps_block, h->delta, h->occ_list, h->group_count,
                     h->col_count, h->chunk_tot, h->export_buf, h->pts_in, h->world, h->valid, h->k0, h->v0, h->k1, h->v1,
                     h->hist, h->blk, h->seg_key, h->seg_start, h->mom, h->part, h->sd, h->diff_rec,
                     h->diff_colh, h->diff_part, h->diff_sums, h->diff_colpt, h->diff_pmark, h->graph_sd, h->rsec, h->rorder, h->azhist, h->grids, h->raw, h->tscratch,
@@ -432,7 +433,8 @@ extern "C" int gvom_create(const gvom_params *params, gvom_handle **out) {
     h->rough = (double *)(h->vis + X);
     CKC(dalloc(&h->delta, X));
     CKC(dalloc(&h->grids, 5 * X));
-    CKC(dalloc(&h->occ_list, V));
+    if (!comb_cells_direct(g)) CKC(dalloc(&h->occ_list, V));
+    CKC(dalloc(&h->group_count, comb_groups(g) + 3));   // read four at a time
     h->col_count_words = gvom_plan::alloc_col_count_words(X);
     CKC(dalloc(&h->col_count, h->col_count_words));
     CKC(dalloc(&h->occ_bits, X * ((g.Z + 63) / 64)));
@@ -1235,13 +1237,13 @@ static int combine_impl(gvom_handle *h, uint8_t *host_maps = nullptr) {
     if (h->capturing) h->cap_ops.push_back(-1);
     const int cur = 1 - h->parity;
     stage_event(h, 5);
-    CKH(h, launch_comb_tables(g, h->st, h->slot_tables, h->zero_page, h->comb_tables, h->col_count, h->occ_bits,
-                              h->height, h->inferred, st));
+    CKH(h, launch_comb_tables(g, h->st, h->slot_tables, h->zero_page, h->comb_tables, h->col_count, h->group_count,
+                              comb_groups(g), h->occ_bits, h->height, h->inferred, st));
     stage_event(h, 6);
-    CKH(h, launch_scan_columns(h->col_count, h->col_count_words, g.X, h->chunk_tot, h->chunk_tot_words, h->st, st));
     CKH(h, join_metrics(h));   // the record merge reads the newest stage's metrics
-    CKH(h, launch_comb_records(g, h->st, h->slot_tables, h->slot_recs, h->ncap, h->comb_tables, h->comb_recs,
-                               h->ccap, h->col_count, h->chunk_tot, h->occ_bits, h->occ_list, h->height, st));
+    CKH(h, launch_comb_cells(g, h->st, h->slot_tables, h->slot_recs, h->ncap, h->comb_tables, h->comb_recs, h->ccap,
+                             h->col_count, h->col_count_words, h->group_count, h->chunk_tot, h->chunk_tot_words,
+                             h->occ_bits, h->occ_list, h->height, st));
     stage_event(h, 7);
     CKH(h, launch_maps2d(g, h->st, h->height, h->inferred, h->comb_tables, h->comb_recs, h->ccap, h->slope_x,
                          h->slope_y, h->rough, h->delta, h->pos, h->neg, h->vis, host_maps, st));

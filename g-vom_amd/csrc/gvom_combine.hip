@@ -9,17 +9,16 @@
 //             the column's occupied count.
 //   scan      exclusive scan of the column counts -> first cell id of each column,
 //             so ids follow the z-contiguous voxel order (a legal permutation of the
-//             reference's atomic order).
-//   records   one wavefront per column: assign ids, merge the sources' records in
+//             reference's atomic order); large maps only.
+//   cells     one thread per occupied voxel: its id, the sources' records merged in
 //             slot order then the previous map (gvom.py:889-980), eigenvalues
-//             (1424-1487), and the column passes: height (561-576), inferred height
-//             (580-590), positive-obstacle density window (530-555).
+//             (1424-1487), heights (561-576).
 //   maps2d    16x16 column tiles with a 15-cell halo in LDS: slope and roughness
 //             (718-805), guessed height delta (593-714), positive/negative obstacle
 //             and visibility maps (445-555).
-//   commit    ping-pong parity of the combined buffers, flipped by the column scan's
-//             first thread (every later kernel of the combine reads the new parity), and
-//             the new map's cell count, written by the record merge.
+//   commit    ping-pong parity of the combined buffers, set by the cell pass as
+//             parity_next and made the parity by the 2D maps, and the new map's cell
+//             count, written by the cell pass.
 #include <hip/hip_runtime.h>
 
 #include "gvom_kernels.h"
@@ -34,22 +33,6 @@ __device__ __forceinline__ float py_maxf(float a, float b) { return (b > a) ? b 
 __device__ __forceinline__ float py_minf(float a, float b) { return (b < a) ? b : a; }
 __device__ __forceinline__ double py_max(double a, double b) { return (b > a) ? b : a; }
 __device__ __forceinline__ double py_min(double a, double b) { return (b < a) ? b : a; }
-
-struct SrcCol {
-    const int32_t *col;   // source column base (nullptr when the shifted column is off-map)
-    int32_t dz;
-};
-
-__device__ __forceinline__ SrcCol source_column(const int32_t *table, const double co[3], const double so[3],
-                                                int64_t x, int64_t y, const Geo &g) {
-    SrcCol r;
-    int64_t dx = (int64_t)(co[0] - so[0]), dy = (int64_t)(co[1] - so[1]);
-    r.dz = (int32_t)(co[2] - so[2]);
-    int64_t ux = x + dx, uy = y + dy;
-    if (ux < 0 || ux >= g.XY || uy < 0 || uy >= g.XY) r.col = nullptr;
-    else r.col = table + (ux * g.XY + uy) * g.Z;
-    return r;
-}
 
 // ------------------------------------------------------------------------------------
 // Table pass.  A wavefront combines cpw consecutive columns, zl lanes per column, eight
@@ -94,11 +77,13 @@ __global__ __launch_bounds__(256) void k_comb_tables(Geo g, const DevState *__re
                                                      const int32_t *__restrict__ zero_page,
                                                      int32_t *__restrict__ comb_tables,
                                                      int32_t *__restrict__ col_count,
-                                                     uint64_t *__restrict__ occ_bits, double *__restrict__ height,
-                                                     double *__restrict__ inferred, int zl, int cpw) {
+                                                     int32_t *__restrict__ group, uint64_t *__restrict__ occ_bits,
+                                                     double *__restrict__ height, double *__restrict__ inferred,
+                                                     int zl, int cpw) {
     // per wavefront: a byte of occupied and a byte of free bits (passes, no hit) per lane, as
     // 64-bit words of its columns
     __shared__ __align__(16) uint8_t occ_b[4][512], free_b[4][512];
+    __shared__ uint32_t wave_cells[4];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int32_t XY = g.XY, Z = g.Z, X = (int32_t)g.X;
     const int NW = (Z + 63) >> 6;   // occupancy words per column
@@ -202,8 +187,8 @@ __global__ __launch_bounds__(256) void k_comb_tables(Geo g, const DevState *__re
     __syncthreads();
     // one lane per column
     const int32_t cc = c0 + lane;
+    uint32_t cnt = 0;
     if (lane < cpw && cc < X) {
-        uint32_t cnt = 0;
         int ff = -1;
         for (int w = 0; w < NW; ++w) {
             const uint64_t o = reinterpret_cast<const uint64_t *>(occ_b[wv])[lane * NW + w];
@@ -227,32 +212,25 @@ __global__ __launch_bounds__(256) void k_comb_tables(Geo g, const DevState *__re
             height[cc] = h;
         }
     }
+    // the block's occupied voxels
+    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off);
+    if (lane == 0) wave_cells[wv] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        group[blockIdx.x] = (int32_t)(wave_cells[0] + wave_cells[1] + wave_cells[2] + wave_cells[3]);
 }
 
 // ------------------------------------------------------------------------------------
 // Column id scan: blocks of 1024 threads scan COLSCAN consecutive column counts in place
-// (exclusive, int4 loads) and write their total; k_comb_records adds the totals of the
+// (exclusive, int4 loads) and write their total; k_comb_ids adds the totals of the
 // earlier chunks.
 constexpr int COLSCAN = gvom_plan::COLSCAN;   // 1024 threads x 4 columns
 static_assert(COLSCAN == 1024 * 4, "column scan: 1024 threads x 4 columns per block");
 
 __global__ __launch_bounds__(1024) void k_col_scan(int32_t *__restrict__ cnt, int64_t X,
-                                                   int32_t *__restrict__ chunk_tot, DevState *__restrict__ st) {
+                                                   int32_t *__restrict__ chunk_tot) {
     __shared__ int32_t wsum[16];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    if (blockIdx.x == 0 && t == 0) {
-        // origin of the combined map being built = newest slot's origin (gvom.py:229), and
-        // the ping-pong flip (gvom.py:276-316): no other thread of this kernel reads the
-        // parity, the combine's earlier kernel (the table pass) has finished, and its later
-        // kernels read the new value
-        const int cur = 1 - st->parity;
-        const double *co = st->slot_origin[st->last_slot];
-        st->comb_origin[cur][0] = co[0];
-        st->comb_origin[cur][1] = co[1];
-        st->comb_origin[cur][2] = co[2];
-        st->parity = cur;
-        st->have_last = 1;
-    }
     const int64_t i = (int64_t)blockIdx.x * COLSCAN + 4 * t;
     // four counts per thread; past the last column they read as 0 and are not written
     int4 v = make_int4(0, 0, 0, 0);
@@ -289,27 +267,50 @@ __global__ __launch_bounds__(1024) void k_col_scan(int32_t *__restrict__ cnt, in
 }
 
 // ------------------------------------------------------------------------------------
+// Division of several f64 numbers by one divisor, each quotient rounded as a / b rounds it.  With
+// r = 1 / b correctly rounded, one correction of a r leaves a quotient within an ulp and the next
+// rounds it correctly (Markstein, IBM J. Res. Dev. 34(1), 1990), as long as the remainders do
+// not underflow; here b is a count of points and |a| far from the ends of the range.  Five
+// full-rate instructions instead of a division's scaling, quarter-rate reciprocal and fix-up.
+struct DivideBy {
+    double b, r;
+    __device__ __forceinline__ explicit DivideBy(double d) : b(d), r(1.0 / d) {}
+    __device__ __forceinline__ double operator()(double a) const {
+        double q = a * r;
+        q = fma(fma(-b, q, a), r, q);
+        return fma(fma(-b, q, a), r, q);
+    }
+};
+struct DivideByF {
+    float b;
+    __device__ __forceinline__ explicit DivideByF(float d) : b(d) {}
+    __device__ __forceinline__ float operator()(float a) const { return a / b; }
+};
+template <typename T> struct DivideOf { using type = DivideByF; };
+template <> struct DivideOf<double> { using type = DivideBy; };
+
 // Record merge, __combine_metrics (gvom.py:889-980) with Numba's typing: the product of
 // two combined (f32) entries is f32, everything touching an f64 operand is f64.
 template <typename OT>
 __device__ __forceinline__ void merge_record(float cm[10], int32_t &hit, int32_t &tot, float &mh, const OT om[10],
                                              int32_t ohit, int32_t otot, float omh) {
     using MT = decltype((float)0 * (OT)0);
-    MT mx = (cm[0] * cm[9] + om[0] * om[9]) / (cm[9] + om[9]);
-    MT my = (cm[1] * cm[9] + om[1] * om[9]) / (cm[9] + om[9]);
-    MT mz = (cm[2] * cm[9] + om[2] * om[9]) / (cm[9] + om[9]);
-    float c3 = (float)((cm[9] * cm[3] + om[9] * om[3] + cm[9] * (cm[0] - mx) * (cm[0] - mx) +
-                        om[9] * (om[0] - mx) * (om[0] - mx)) / (cm[9] + om[9]));
-    float c4 = (float)((cm[9] * cm[4] + om[9] * om[4] + cm[9] * (cm[0] - mx) * (cm[1] - my) +
-                        om[9] * (om[0] - mx) * (om[1] - my)) / (cm[9] + om[9]));
-    float c5 = (float)((cm[9] * cm[5] + om[9] * om[5] + cm[9] * (cm[0] - mx) * (cm[2] - mz) +
-                        om[9] * (om[0] - mx) * (om[2] - mz)) / (cm[9] + om[9]));
-    float c6 = (float)((cm[9] * cm[6] + om[9] * om[6] + cm[9] * (cm[1] - my) * (cm[1] - my) +
-                        om[9] * (om[1] - my) * (om[1] - my)) / (cm[9] + om[9]));
-    float c7 = (float)((cm[9] * cm[7] + om[9] * om[7] + cm[9] * (cm[1] - my) * (cm[2] - mz) +
-                        om[9] * (om[1] - my) * (om[2] - mz)) / (cm[9] + om[9]));
-    float c8 = (float)((cm[9] * cm[8] + om[9] * om[8] + cm[9] * (cm[2] - mz) * (cm[2] - mz) +
-                        om[9] * (om[2] - mz) * (om[2] - mz)) / (cm[9] + om[9]));
+    const typename DivideOf<MT>::type by(cm[9] + om[9]);
+    MT mx = by(cm[0] * cm[9] + om[0] * om[9]);
+    MT my = by(cm[1] * cm[9] + om[1] * om[9]);
+    MT mz = by(cm[2] * cm[9] + om[2] * om[9]);
+    float c3 = (float)by(cm[9] * cm[3] + om[9] * om[3] + cm[9] * (cm[0] - mx) * (cm[0] - mx) +
+                         om[9] * (om[0] - mx) * (om[0] - mx));
+    float c4 = (float)by(cm[9] * cm[4] + om[9] * om[4] + cm[9] * (cm[0] - mx) * (cm[1] - my) +
+                         om[9] * (om[0] - mx) * (om[1] - my));
+    float c5 = (float)by(cm[9] * cm[5] + om[9] * om[5] + cm[9] * (cm[0] - mx) * (cm[2] - mz) +
+                         om[9] * (om[0] - mx) * (om[2] - mz));
+    float c6 = (float)by(cm[9] * cm[6] + om[9] * om[6] + cm[9] * (cm[1] - my) * (cm[1] - my) +
+                         om[9] * (om[1] - my) * (om[1] - my));
+    float c7 = (float)by(cm[9] * cm[7] + om[9] * om[7] + cm[9] * (cm[1] - my) * (cm[2] - mz) +
+                         om[9] * (om[1] - my) * (om[2] - mz));
+    float c8 = (float)by(cm[9] * cm[8] + om[9] * om[8] + cm[9] * (cm[2] - mz) * (cm[2] - mz) +
+                         om[9] * (om[2] - mz) * (om[2] - mz));
     cm[3] = c3; cm[4] = c4; cm[5] = c5; cm[6] = c6; cm[7] = c7; cm[8] = c8;
     cm[0] = (float)mx; cm[1] = (float)my; cm[2] = (float)mz;
     cm[9] = (float)(cm[9] + om[9]);
@@ -347,13 +348,224 @@ __device__ __forceinline__ void eigen3(const float m[10], float ev[3]) {
     }
 }
 
-// Cell ids: one wavefront per column assigns ids in z order (first id of the column =
+// State of the combined map being built, by one thread: its origin = the newest slot's
+// (gvom.py:229), and the ping-pong flip (gvom.py:276-316): no other thread before the next
+// kernel reads these, and the 2D maps make parity_next the parity once no kernel of the combine
+// reads the old one.
+__device__ __forceinline__ void begin_map(DevState *st, int cur) {
+    const double *co = st->slot_origin[st->last_slot];
+    st->comb_origin[cur][0] = co[0];
+    st->comb_origin[cur][1] = co[1];
+    st->comb_origin[cur][2] = co[2];
+    st->parity_next = cur;
+    st->have_last = 1;
+}
+
+// k-th (from 0) set bit of m.
+__device__ __forceinline__ int select_bit(uint64_t m, int k) {
+    int at = 0;
+    uint32_t h = (uint32_t)m;
+    int n = __popc(h);
+    if (k >= n) {
+        k -= n;
+        at = 32;
+        h = (uint32_t)(m >> 32);
+    }
+#pragma unroll
+    for (int w = 16; w > 0; w >>= 1) {
+        n = __popc(h & ((1u << w) - 1u));
+        if (k >= n) {
+            k -= n;
+            at += w;
+            h >>= w;
+        }
+    }
+    return at;
+}
+
+// Record merge of one cell of the combined map (lin: its table index, mask: its sources) and its
+// eigenvalues: sources in slot order, then the previous combined map (gvom.py:280-298).  Per
+// group of MERGE_GROUP slots, all source-table loads are issued, then all record loads, then
+// the merges run in order, so a thread has a group's gathers in flight together.
+constexpr int MERGE_GROUP = 4;
+
+__device__ __forceinline__ void merge_cell(const Geo &g, const DevState *__restrict__ st,
+                                           const int32_t *__restrict__ slot_tables,
+                                           const SlotRec *__restrict__ slot_recs, int64_t ncap,
+                                           const int32_t *__restrict__ ltab, const CombRec *__restrict__ lrec, int flip,
+                                           int parity, const double *__restrict__ co, int64_t lin, uint32_t mask,
+                                           CombRec &out) {
+    float cm[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    int32_t hit = 0, tot = 0;
+    float mh = 1.0f;
+    for (int s0 = 0; s0 < g.B; s0 += MERGE_GROUP) {
+        uint32_t sid[MERGE_GROUP];
+        bool use[MERGE_GROUP];
+#pragma unroll
+        for (int q = 0; q < MERGE_GROUP; ++q) {
+            const int s = s0 + q;
+            use[q] = s < g.B && ((mask >> s) & 1u);
+            const int32_t *addr = slot_tables;   // any valid word when the source is unused
+            if (use[q]) {
+                const int4 sh = *reinterpret_cast<const int4 *>(st->comb_shift[s]);
+                addr = slot_tables + (int64_t)cur_buf(flip, s) * g.V + lin +
+                       ((int64_t)sh.x * g.XY + sh.y) * g.Z + sh.z;
+            }
+            sid[q] = (uint32_t)*addr & MASK31;
+        }
+        SlotRec rec[MERGE_GROUP];
+#pragma unroll
+        for (int q = 0; q < MERGE_GROUP; ++q)
+            rec[q] = slot_recs[(int64_t)cur_buf(flip, use[q] ? s0 + q : 0) * ncap + (use[q] ? sid[q] : 0)];
+#pragma unroll
+        for (int q = 0; q < MERGE_GROUP; ++q)
+            if (use[q]) merge_record<double>(cm, hit, tot, mh, rec[q].m, rec[q].hit, rec[q].total, rec[q].min_h);
+    }
+    if (mask & (1u << LAST_BIT)) {
+        const double *lo = st->comb_origin[parity];
+        const int64_t dx = (int64_t)(co[0] - lo[0]), dy = (int64_t)(co[1] - lo[1]), dz = (int64_t)(co[2] - lo[2]);
+        const uint32_t lid = (uint32_t)ltab[lin + (dx * g.XY + dy) * g.Z + dz] & MASK31;
+        const CombRec &q = lrec[lid];
+        merge_record<float>(cm, hit, tot, mh, q.m, q.hit, q.total, q.min_h);
+    }
+    out.hit = hit;
+    out.total = tot;
+    out.min_h = mh;
+#pragma unroll
+    for (int j = 0; j < 10; ++j) out.m[j] = cm[j];
+    eigen3(cm, out.ev);
+}
+
+// Cells of CELL_PARTS x 64 columns per block: ids in z order from each part's first id (the
+// occupied voxels of all columns before it), the table entry becomes OCC | id, and the record
+// merge of the cell: sources in slot order, then the previous combined map (gvom.py:280-298).
+// A thread finds its cell from the columns' occupancy words (prefix of their counts, then the
+// k-th bit), so no list of cells goes through memory.  The parts lie a CELL_PARTS-th of the map
+// apart: the cells crowd around the sensor, and a block of neighbouring columns there would
+// set the time.  The thread holding a column's lowest occupied voxel writes its height
+// (min_h + z + oz) * z_res (gvom.py:572-576).
+//
+// The first id: the block adds the table pass's counts of occupied voxels per group of gcols
+// columns (four per load, several loads in flight: one after another they set the time).
+//
+// Bound by latency: a cell is a chain of table word -> source words -> records, twice for eight
+// slots, and the merges between them.  256 x 256 x 64, 8 slots, 38k cells: 16.6 us, where the
+// column scan, the ids with their list and the merge of the list took 4.7 + 5.3 + 14.5.
+constexpr int CELL_PARTS = 4;          // groups of 64 columns per block
+constexpr int CELL_THREADS = 256;
+
+__global__ __launch_bounds__(CELL_THREADS) void k_comb_cells(
+    Geo g, DevState *__restrict__ st, const int32_t *__restrict__ slot_tables, const SlotRec *__restrict__ slot_recs,
+    int64_t ncap, int32_t *__restrict__ comb_tables, CombRec *__restrict__ comb_recs, int64_t ccap,
+    const int32_t *__restrict__ col_count, const int32_t *__restrict__ group, int gcols,
+    const uint64_t *__restrict__ occ_bits, double *__restrict__ height) {
+    constexpr int COLS = 64 * CELL_PARTS, WAVES = CELL_THREADS / 64, PER = WAVES / CELL_PARTS;
+    __shared__ uint64_t occ[COLS * 4];
+    __shared__ uint32_t pre[COLS + 1];
+    __shared__ uint32_t part[WAVES];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int NW = (g.Z + 63) >> 6;
+    const int32_t X = (int32_t)g.X;
+    const int parity = st->parity, cur = 1 - parity, flip = st->flip;
+    // origin of the combined map being built = newest slot's (gvom.py:229)
+    const double *co = st->slot_origin[st->last_slot];
+    if (blockIdx.x == 0 && t == 0) begin_map(st, cur);
+    // part p of the block: the 64 columns from first_column(p) on
+    auto first_column = [&](int p) { return ((int32_t)blockIdx.x + p * (int32_t)gridDim.x) * 64; };
+    if (t < COLS) {
+        const int32_t c = first_column(w) + lane;
+        uint32_t n = 0;
+        for (int q = 0; q < NW; ++q) {
+            const uint64_t o = c < X ? occ_bits[(int64_t)c * NW + q] : 0ull;
+            occ[t * NW + q] = o;
+            n += __popcll(o);
+        }
+        uint32_t v = n;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t u = __shfl_up(v, off);
+            if (lane >= off) v += u;
+        }
+        pre[t + 1] = v;
+        if (t == 0) pre[0] = 0;
+    }
+    {
+        // first id of part w / PER, its terms shared by PER wavefronts
+        const int32_t c0 = first_column(w / PER);
+        const int at = (w % PER) * 64 + lane;
+        uint32_t base = 0;
+        if (c0 < X) {
+            const int32_t ng = c0 / gcols;
+            // four counts per load and several loads in flight (the last load may run past ng: the
+            // counts are padded)
+            const int4 *g4 = reinterpret_cast<const int4 *>(group);
+#pragma unroll 4
+            for (int32_t k = at; k < (ng + 3) / 4; k += 64 * PER) {
+                const int4 v = g4[k];
+                base += (uint32_t)v.x + (4 * k + 1 < ng ? (uint32_t)v.y : 0u) + (4 * k + 2 < ng ? (uint32_t)v.z : 0u) +
+                        (4 * k + 3 < ng ? (uint32_t)v.w : 0u);
+            }
+            for (int32_t c = ng * gcols + at; c < c0; c += 64 * PER) base += (uint32_t)col_count[c];
+        }
+        for (int off = 32; off > 0; off >>= 1) base += __shfl_xor(base, off);
+        if (lane == 0) part[w] = base;
+    }
+    __syncthreads();
+    {
+        // prefixes within each part -> within the block
+        uint32_t add = 0;
+        if (t < COLS)
+            for (int q = 1; q <= w; ++q) add += pre[64 * q];
+        __syncthreads();
+        if (t < COLS) pre[t + 1] += add;
+        __syncthreads();
+    }
+    const uint32_t n = pre[COLS];
+    auto first_id = [&](int p) {   // minus the block's cells before the part
+        uint32_t v = part[p * PER];
+        for (int q = 1; q < PER; ++q) v += part[p * PER + q];
+        return v - pre[64 * p];
+    };
+    if (t < CELL_PARTS && first_column(t) < X && first_column(t) + 64 >= X) {
+        // the new map's cell count (the commit of gvom.py:276-316)
+        const int32_t total = (int32_t)(first_id(t) + pre[64 * (t + 1)]);
+        st->comb_cells[cur] = total;
+        st->comb_total = total;
+    }
+    CombRec *crec = comb_recs + (int64_t)cur * ccap;
+    const CombRec *lrec = comb_recs + (int64_t)parity * ccap;
+    int32_t *ctab = comb_tables + (int64_t)cur * g.V;
+    const int32_t *ltab = comb_tables + (int64_t)parity * g.V;
+    for (uint32_t k = t; k < n; k += CELL_THREADS) {
+        // the cell's column: the last one whose first cell is at or before k
+        int cl = 0;
+#pragma unroll
+        for (int step = COLS / 2; step > 0; step >>= 1)
+            if (pre[cl + step] <= k) cl += step;
+        uint32_t r = k - pre[cl];
+        const bool lowest = r == 0;
+        int zw = 0;
+        uint64_t o = occ[cl * NW];
+        while (r >= (uint32_t)__popcll(o)) {
+            r -= __popcll(o);
+            o = occ[cl * NW + ++zw];
+        }
+        const int64_t z = zw * 64 + select_bit(o, (int)r);
+        const int64_t c = first_column(cl >> 6) + (cl & 63);
+        const int64_t lin = c * g.Z + z;
+        const uint32_t id = first_id(cl >> 6) + k;
+        const uint32_t mask = (uint32_t)ctab[lin] & MASK31;
+        ctab[lin] = (int32_t)(GVOM_OCC | id);
+        CombRec out;
+        merge_cell(g, st, slot_tables, slot_recs, ncap, ltab, lrec, flip, parity, co, lin, mask, out);
+        if ((int64_t)id < ccap) crec[id] = out;   // the records hold ccap cells
+        if (lowest) height[c] = (((double)out.min_h + (double)z) + co[2]) * g.z_res;
+    }
+}
+
+// Cell ids of a large map: one lane per column assigns ids in z order (first id of the column =
 // earlier chunks' totals + in-chunk exclusive prefix), rewrites the table entry to
-// OCC | id and appends (voxel, source mask) to the compact list.  It also writes the
-// inferred height (lowest free voxel, gvom.py:580-590) and, for columns without an
-// occupied voxel, the height-map default (robot-radius cell corner, gvom.py:561-570).
-// Bit 31 of the list's voxel word marks the lowest occupied voxel of a column.
-__global__ __launch_bounds__(256) void k_comb_ids(Geo g, const DevState *__restrict__ st,
+// OCC | id and appends (voxel, source mask) to the compact list.  Bit 31 of the list's voxel word marks the lowest occupied voxel of a column.
+__global__ __launch_bounds__(256) void k_comb_ids(Geo g, DevState *__restrict__ st,
                                                   int32_t *__restrict__ comb_tables,
                                                   const int32_t *__restrict__ col_base,
                                                   const int32_t *__restrict__ chunk_tot,
@@ -365,7 +577,8 @@ __global__ __launch_bounds__(256) void k_comb_ids(Geo g, const DevState *__restr
     const int32_t X = (int32_t)g.X, Z = g.Z;
     const int32_t cb = uni((int32_t)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64);
     if (cb >= X) return;
-    const int cur = st->parity;   // flipped by the column scan
+    const int cur = 1 - st->parity;
+    if (cb == 0 && lane == 0) begin_map(st, cur);
     const int NW = (Z + 63) >> 6;
     int32_t *ctab = comb_tables + (int64_t)cur * g.V;
     // earlier chunks' totals (a wavefront's 64 columns lie in one chunk: 64 divides COLSCAN)
@@ -394,14 +607,8 @@ __global__ __launch_bounds__(256) void k_comb_ids(Geo g, const DevState *__restr
     }
 }
 
-// Record merge per occupied voxel of the compact list (grid-stride).  Sources are taken
-// in slot order, then the previous combined map (gvom.py:280-298).  Per group of
-// MERGE_GROUP slots, all source-table loads are issued, then all record loads, then the
-// merges run in order, so a thread has a group's gathers in flight together.  The
-// thread holding a column's lowest occupied voxel writes its height
-// (min_h + z + oz) * z_res (gvom.py:572-576).
-constexpr int MERGE_GROUP = 4;
-
+// Record merge per occupied voxel of the compact list (grid-stride) of a large map.  The thread
+// holding a column's lowest occupied voxel writes its height.
 __global__ __launch_bounds__(256) void k_comb_merge(Geo g, DevState *__restrict__ st,
                                                     const int32_t *__restrict__ slot_tables,
                                                     const SlotRec *__restrict__ slot_recs, int64_t ncap,
@@ -410,7 +617,7 @@ __global__ __launch_bounds__(256) void k_comb_merge(Geo g, DevState *__restrict_
                                                     const uint2 *__restrict__ occ_list,
                                                     const int32_t *__restrict__ chunk_tot, int64_t nchunk,
                                                     double *__restrict__ height) {
-    const int cur = st->parity, parity = 1 - cur, flip = st->flip;   // flipped by the column scan
+    const int cur = st->parity_next, parity = 1 - cur, flip = st->flip;
     const double *co = st->comb_origin[cur];
     const int lane = threadIdx.x & 63;
     uint32_t C = 0;
@@ -428,50 +635,14 @@ __global__ __launch_bounds__(256) void k_comb_merge(Geo g, DevState *__restrict_
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; id < (int64_t)C; id += stride) {
         const uint2 e = occ_list[id];
-        const uint32_t lin = e.x & MASK31, mask = e.y;
-        const bool lowest = (e.x >> 31) != 0;
-        const int64_t z = lin % g.Z, c = lin / g.Z, x = c / g.XY, y = c % g.XY;
-        float cm[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        int32_t hit = 0, tot = 0;
-        float mh = 1.0f;
-        for (int s0 = 0; s0 < g.B; s0 += MERGE_GROUP) {
-            uint32_t sid[MERGE_GROUP];
-            bool use[MERGE_GROUP];
-#pragma unroll
-            for (int k = 0; k < MERGE_GROUP; ++k) {
-                const int s = s0 + k;
-                use[k] = s < g.B && ((mask >> s) & 1u);
-                const int32_t *addr = slot_tables;   // any valid word when the source is unused
-                if (use[k]) {
-                    SrcCol sc = source_column(slot_tables + (int64_t)cur_buf(flip, s) * g.V, co, st->slot_origin[s],
-                                              x, y, g);
-                    addr = sc.col + z + sc.dz;
-                }
-                sid[k] = (uint32_t)*addr & MASK31;
-            }
-            SlotRec r[MERGE_GROUP];
-#pragma unroll
-            for (int k = 0; k < MERGE_GROUP; ++k)
-                r[k] = slot_recs[(int64_t)cur_buf(flip, use[k] ? s0 + k : 0) * ncap + (use[k] ? sid[k] : 0)];
-#pragma unroll
-            for (int k = 0; k < MERGE_GROUP; ++k)
-                if (use[k]) merge_record<double>(cm, hit, tot, mh, r[k].m, r[k].hit, r[k].total, r[k].min_h);
-        }
-        if (mask & (1u << LAST_BIT)) {
-            SrcCol sc = source_column(ltab, co, st->comb_origin[parity], x, y, g);
-            const uint32_t lid = (uint32_t)sc.col[z + sc.dz] & MASK31;
-            const CombRec &r = lrec[lid];
-            merge_record<float>(cm, hit, tot, mh, r.m, r.hit, r.total, r.min_h);
-        }
+        const uint32_t lin = e.x & MASK31;
         CombRec out;
-        out.hit = hit;
-        out.total = tot;
-        out.min_h = mh;
-#pragma unroll
-        for (int j = 0; j < 10; ++j) out.m[j] = cm[j];
-        eigen3(cm, out.ev);
+        merge_cell(g, st, slot_tables, slot_recs, ncap, ltab, lrec, flip, parity, co, lin, e.y, out);
         crec[id] = out;
-        if (lowest) height[c] = (((double)mh + (double)z) + co[2]) * g.z_res;
+        if (e.x >> 31) {
+            const uint32_t c = lin / (uint32_t)g.Z, z = lin - c * (uint32_t)g.Z;
+            height[c] = (((double)out.min_h + (double)z) + co[2]) * g.z_res;
+        }
     }
 }
 
@@ -497,7 +668,7 @@ __device__ __forceinline__ int first_in(uint64_t m, int lo, int hi) {
 // three latency chains overlap; the first group then writes the maps.  (With the slope fit
 // and the ring search on the same threads the kernel took 21.0 us on 256 x 256 cells, event
 // timed; skipping either shortened it by 3.7 and 6.6 us.)
-__global__ __launch_bounds__(MT) void k_maps2d(Geo g, const DevState *__restrict__ st,
+__global__ __launch_bounds__(MT) void k_maps2d(Geo g, DevState *__restrict__ st,
                                                 const double *__restrict__ height,
                                                 const double *__restrict__ inferred,
                                                 const int32_t *__restrict__ comb_tables,
@@ -512,6 +683,9 @@ __global__ __launch_bounds__(MT) void k_maps2d(Geo g, const DevState *__restrict
     __shared__ int32_t winpv[TT];   // window density result per column of the tile
     __shared__ double dhw[TT];      // guessed-height difference per column of the tile
     const int XY = g.XY;
+    const int cur = st->parity_next;
+    // the flip set by the cell pass: nothing else in this kernel reads the parity
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) st->parity = cur;
     const int bx = blockIdx.y * TILE, by = blockIdx.x * TILE;   // tile origin (x rows, y fastest)
     for (int k = threadIdx.x; k < LT * LT; k += MT) {
         int lx = k / LT, ly = k % LT;
@@ -549,7 +723,6 @@ __global__ __launch_bounds__(MT) void k_maps2d(Geo g, const DevState *__restrict
         int32_t pvw = 0;
         if (act) {
             const double h0 = HAT(x0, y0);
-            const int cur = st->parity;   // flipped by the column scan
             const double oz = st->comb_origin[cur][2];
             const double flo = floor(((h0 + g.pos_thr) / g.z_res) - oz);
             const double fhi = floor(((h0 + g.robot_h) / g.z_res) - oz);
@@ -814,38 +987,62 @@ inline unsigned nblocks(int64_t n, int per) { return (unsigned)((n + per - 1) / 
 
 int64_t zero_page_words() { return ZERO_PAGE_WORDS; }
 
+static int table_lanes(const Geo &g) { return (g.Z + ZPL - 1) / ZPL; }
+
+int64_t comb_group_columns(const Geo &g) { return 4 * (64 / table_lanes(g)); }
+int64_t comb_groups(const Geo &g) { return (g.X + comb_group_columns(g) - 1) / comb_group_columns(g); }
+
 hipError_t launch_comb_tables(const Geo &g, DevState *st, const int32_t *slot_tables, const int32_t *zero_page,
-                              int32_t *comb_tables, int32_t *col_count, uint64_t *occ_bits, double *height,
-                              double *inferred, hipStream_t s) {
-    const int zl = (g.Z + ZPL - 1) / ZPL, cpw = 64 / zl;
-    k_comb_tables<<<nblocks(g.X, 4 * cpw), 256, 0, s>>>(g, st, slot_tables, zero_page, comb_tables, col_count, occ_bits,
-                                                        height, inferred, zl, cpw);
+                              int32_t *comb_tables, int32_t *col_count, int32_t *group, int64_t group_words,
+                              uint64_t *occ_bits, double *height, double *inferred, hipStream_t s) {
+    if (comb_groups(g) > group_words) return hipErrorInvalidValue;
+    const int zl = table_lanes(g);
+    k_comb_tables<<<(unsigned)comb_groups(g), 256, 0, s>>>(g, st, slot_tables, zero_page, comb_tables, col_count, group,
+                                                           occ_bits, height, inferred, zl, 64 / zl);
     return hipGetLastError();
 }
 
 int64_t col_chunks(int64_t X) { return gvom_plan::col_chunks(X); }
 
+// The parity and the other device state stay as they are (the cell pass sets them).
 hipError_t launch_scan_columns(int32_t *col_count, int64_t count_words, int64_t X, int32_t *chunk_tot,
-                               int64_t chunk_words, DevState *st, hipStream_t s) {
+                               int64_t chunk_words, DevState *, hipStream_t s) {
     if (X < 1 || gvom_plan::col_scan_count_words(X) > count_words || gvom_plan::col_scan_chunk_words(X) > chunk_words)
         return hipErrorInvalidValue;
-    k_col_scan<<<(unsigned)col_chunks(X), 1024, 0, s>>>(col_count, X, chunk_tot, st);
+    k_col_scan<<<(unsigned)col_chunks(X), 1024, 0, s>>>(col_count, X, chunk_tot);
     return hipGetLastError();
 }
 
-hipError_t launch_comb_records(const Geo &g, DevState *st, const int32_t *slot_tables,
-                               const SlotRec *slot_recs, int64_t ncap, int32_t *comb_tables,
-                               CombRec *comb_recs, int64_t ccap, const int32_t *col_base,
-                               const int32_t *chunk_tot, const uint64_t *occ_bits, uint2 *occ_list, double *height,
-                               hipStream_t s) {
-    k_comb_ids<<<nblocks((g.X + 63) / 64, 4), 256, 0, s>>>(g, st, comb_tables, col_base, chunk_tot, occ_bits,
-                                                                 occ_list);
+// Maps of up to this many columns (256 x 256: one block of k_comb_cells per compute unit) merge
+// their cells there; larger ones run the column scan, k_comb_ids and k_comb_merge.  Measured
+// (rocprof, the kernels' sum): 65,536 columns 16.6 against 23.9 us, 22,801 11.5 against 18.9,
+// 4,096 8.1 against 15.2; but 102,400 columns 31 against 27, 160,000 55 against 47.
+constexpr int64_t CELL_MAX_COLUMNS = 65536;
+
+bool comb_cells_direct(const Geo &g) { return g.X <= CELL_MAX_COLUMNS; }
+
+hipError_t launch_comb_cells(const Geo &g, DevState *st, const int32_t *slot_tables, const SlotRec *slot_recs,
+                             int64_t ncap, int32_t *comb_tables, CombRec *comb_recs, int64_t ccap, int32_t *col_count,
+                             int64_t count_words, const int32_t *group, int32_t *chunk_tot, int64_t chunk_words,
+                             const uint64_t *occ_bits, uint2 *occ_list, double *height, hipStream_t s) {
+    if (comb_cells_direct(g)) {
+        static_assert((CELL_PARTS & (CELL_PARTS - 1)) == 0 && CELL_THREADS % (64 * CELL_PARTS) == 0,
+                      "a thread per column, as many wavefronts per part");
+        k_comb_cells<<<nblocks((g.X + 63) / 64, CELL_PARTS), CELL_THREADS, 0, s>>>(
+            g, st, slot_tables, slot_recs, ncap, comb_tables, comb_recs, ccap, col_count, group,
+            (int)comb_group_columns(g), occ_bits, height);
+        return hipGetLastError();
+    }
+    if (!occ_list) return hipErrorInvalidValue;
+    const hipError_t e = launch_scan_columns(col_count, count_words, g.X, chunk_tot, chunk_words, st, s);
+    if (e != hipSuccess) return e;
+    k_comb_ids<<<nblocks((g.X + 63) / 64, 4), 256, 0, s>>>(g, st, comb_tables, col_count, chunk_tot, occ_bits, occ_list);
     k_comb_merge<<<2048, 256, 0, s>>>(g, st, slot_tables, slot_recs, ncap, comb_tables, comb_recs, ccap, occ_list,
                                       chunk_tot, col_chunks(g.X), height);
     return hipGetLastError();
 }
 
-hipError_t launch_maps2d(const Geo &g, const DevState *st, const double *height, const double *inferred,
+hipError_t launch_maps2d(const Geo &g, DevState *st, const double *height, const double *inferred,
                          const int32_t *comb_tables, const CombRec *comb_recs, int64_t ccap, double *slope_x,
                          double *slope_y, double *rough, double *delta, int32_t *pos, int32_t *neg, int32_t *vis,
                          uint8_t *host_maps, hipStream_t s) {

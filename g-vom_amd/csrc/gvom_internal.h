@@ -42,6 +42,7 @@ struct DevState {
     int32_t last_slot;     // gvom.py last_buffer_index
     int32_t filled_mask;   // slots holding a scan
     int32_t parity;        // combined buffer holding the latest combined map
+    int32_t parity_next;   // the one the combine in flight builds, set by its cell pass
     int32_t have_last;     // a previous combined map exists
     int32_t nseg;          // segments of the current process batch
     int32_t nvalid;        // sorted keys != NOKEY in the current process batch
@@ -82,7 +83,7 @@ struct DevState {
 __host__ __device__ __forceinline__ int cur_buf(int32_t flip, int slot) { return 2 * slot + ((flip >> slot) & 1); }
 
 // Counts a block publishes for the later blocks of the same launch (radix-sort passes,
-// segments, cell ids): count | PUB_READY in a word that is zero before the launch.  A block
+// segments): count | PUB_READY in a word that is zero before the launch.  A block
 // publishes before it waits and waits only for lower blocks, which were dispatched before it
 // or are dispatched as other work retires, so every wait ends; the poll bound (about 30 ms
 // with s_sleep 1) only guards against a defect: the waiter then goes on without the count

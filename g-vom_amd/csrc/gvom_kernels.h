@@ -87,19 +87,24 @@ hipError_t launch_commit_process(DevState *st, const ScanDesc *sd, const Geo &g,
 // comb_tables must be readable for TABLE_PAD words before and after.
 constexpr int64_t TABLE_PAD = 64;
 int64_t zero_page_words();
+// group: occupied voxels per group of comb_group_columns(g) consecutive columns.
+int64_t comb_group_columns(const Geo &g);
+int64_t comb_groups(const Geo &g);
 hipError_t launch_comb_tables(const Geo &g, DevState *st, const int32_t *slot_tables, const int32_t *zero_page,
-                              int32_t *comb_tables, int32_t *col_count, uint64_t *occ_bits, double *height,
-                              double *inferred, hipStream_t s);
+                              int32_t *comb_tables, int32_t *col_count, int32_t *group, int64_t group_words,
+                              uint64_t *occ_bits, double *height, double *inferred, hipStream_t s);
 int64_t col_chunks(int64_t X);
 hipError_t launch_scan_columns(int32_t *col_count, int64_t count_words, int64_t X, int32_t *chunk_tot,
                                int64_t chunk_words, DevState *st, hipStream_t s);
-// Cell ids + compact list, then the record merge + eigenvalues + heights of occupied columns.
-hipError_t launch_comb_records(const Geo &g, DevState *st, const int32_t *slot_tables,
-                               const SlotRec *slot_recs, int64_t ncap, int32_t *comb_tables,
-                               CombRec *comb_recs, int64_t ccap, const int32_t *col_base,
-                               const int32_t *chunk_tot, const uint64_t *occ_bits, uint2 *occ_list, double *height,
-                               hipStream_t s);
-hipError_t launch_maps2d(const Geo &g, const DevState *st, const double *height, const double *inferred,
+// Cell ids, record merge + eigenvalues + heights of occupied columns, in one kernel, or for
+// large maps (comb_cells_direct(g) false) the column scan, the ids with the compact list
+// occ_list (V entries; null otherwise) and the merge.
+bool comb_cells_direct(const Geo &g);
+hipError_t launch_comb_cells(const Geo &g, DevState *st, const int32_t *slot_tables, const SlotRec *slot_recs,
+                             int64_t ncap, int32_t *comb_tables, CombRec *comb_recs, int64_t ccap, int32_t *col_count,
+                             int64_t count_words, const int32_t *group, int32_t *chunk_tot, int64_t chunk_words,
+                             const uint64_t *occ_bits, uint2 *occ_list, double *height, hipStream_t s);
+hipError_t launch_maps2d(const Geo &g, DevState *st, const double *height, const double *inferred,
                          const int32_t *comb_tables, const CombRec *comb_recs, int64_t ccap, double *slope_x,
                          double *slope_y, double *rough, double *delta, int32_t *pos, int32_t *neg, int32_t *vis,
                          uint8_t *host_maps, hipStream_t s);

@@ -1,7 +1,8 @@
 """The combine at the sizes where its table and cell passes have their edges, against the oracle.
 
 Heights below, at and past a lane's eight voxels and a 64-bit occupancy word, column counts that
-leave the last wavefront and block partly empty, rings of one slot to past a group of loads, and
+leave the last wavefront and block partly empty or are the last that take the one-kernel cell pass
+(256 x 256) and the first that do not, rings of one slot to past a group of loads, and
 an ego that moves by several voxels in x, y and z between scans, back and forth and far enough
 for slots to leave the map altogether.
 """
@@ -20,7 +21,7 @@ MOVES = [(0, 0, 0), (1, 0, 0), (-3, 2, 1), (0, 0, -1), (5, -7, 3), (0, 0, 0), (-
 
 @pytest.mark.parametrize("xy,z,buffer", [
     (4, 4, 1), (5, 7, 2), (16, 8, 4), (37, 9, 5), (30, 16, 8), (33, 60, 3), (24, 63, 4), (20, 64, 9), (21, 65, 2),
-    (17, 100, 3), (9, 128, 4), (12, 250, 1), (11, 256, 30), (130, 30, 3),
+    (17, 100, 3), (9, 128, 4), (12, 250, 1), (11, 256, 30), (130, 30, 3), (256, 5, 2), (257, 6, 2),
 ])
 def test_combine_shapes(xy, z, buffer):
     import gvom
