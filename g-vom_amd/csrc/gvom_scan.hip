@@ -1625,11 +1625,24 @@ __device__ __forceinline__ int64_t neighbour_segment(int64_t x, int64_t y, int64
 }
 
 // 32 lanes (half a wavefront) per occupied voxel, one lane per neighbour; sums over
-// neighbours are shuffle-tree reductions in a fixed lane order.
+// neighbours are reductions in a fixed lane order.  Within 16 lanes they move through DPP
+// (swapped neighbours, swapped pairs, mirrored halves, mirrored rows: after each step the
+// lanes that were summed hold the same value, so a mirror acts as the next power of two), and
+// only the last step goes through the LDS crossbar, which a shuffle of every step filled (ten
+// f64 sums per voxel): k_metrics 16.2 -> 14.1 us for 12k voxels, 38 -> 31 for 40k.
+template <int CTRL> __device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return v + __hiloint2double(__builtin_amdgcn_mov_dpp(hi, CTRL, 0xF, 0xF, false),
+                                __builtin_amdgcn_mov_dpp(lo, CTRL, 0xF, 0xF, false));
+}
 __device__ __forceinline__ double red32(double v) {
-#pragma unroll
-    for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 32);
-    return v;
+    v = dpp_add<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+    v = dpp_add<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+    v = dpp_add<0x141>(v);   // row_half_mirror
+    v = dpp_add<0x140>(v);   // row_mirror
+    constexpr int XOR16 = 0x401F;
+    return v + __hiloint2double(__builtin_amdgcn_ds_swizzle(__double2hiint(v), XOR16),
+                                __builtin_amdgcn_ds_swizzle(__double2loint(v), XOR16));
 }
 
 __global__ __launch_bounds__(256) void k_metrics(const uint32_t *__restrict__ seg_key,
