@@ -251,15 +251,13 @@ struct gvom_handle {
     int overlap = 0;
     hipStream_t front = nullptr;
     hipEvent_t ev_front = nullptr, ev_back = nullptr;
-    // A stage's commit waits only up to its segment sums (ev_front), which write what the
-    // combine's table pass reads; its neighbourhood metrics (slot records' moments) may still
-    // run, on `front` for an overlapped stage, else on `side`, ending at ev_metrics.
-    // metrics_pending: the main stream has not waited for them yet; the combine waits just
-    // before its record merge, every other call that touches the device at its start
-    // (join_metrics).  metrics_on_side: the last ones ran on `side`, so that an overlapped stage,
-    // which does not follow the main stream, waits for ev_metrics itself.
+    // An overlapped stage's commit waits only up to its segment sums (ev_front), which write
+    // what the combine's table pass reads; its neighbourhood metrics (slot records' moments)
+    // may still run on `front`, ending at ev_metrics.  metrics_pending: the main stream has
+    // not waited for them yet; the combine waits just before its record merge, every other
+    // call that touches the device at its start (join_metrics).
     hipEvent_t ev_metrics = nullptr;
-    bool metrics_pending = false, metrics_on_side = false;
+    bool metrics_pending = false;
     // An overlapped stage inside a capture forks `front` from the main stream and `side` from
     // `front`.  hipStreamEndCapture has crashed on that nested fork under an older HIP runtime
     // than the one this library is built against (torch bundles one, and when torch is imported
@@ -281,8 +279,8 @@ struct gvom_handle {
         }                                                                            \
     } while (0)
 
-// Orders the main stream after the neighbourhood metrics a scan stage left running on `front`
-// or `side`.
+// Orders the main stream after the neighbourhood metrics an overlapped scan stage left
+// running on `front`.
 static hipError_t join_metrics(gvom_handle *h) {
     if (!h->metrics_pending) return hipSuccess;
     h->metrics_pending = false;
@@ -511,7 +509,6 @@ static int ensure_capacity(gvom_handle *h, int64_t max_scan, int64_t batch_pts) 
     if (batch_pts < 1) batch_pts = 1;
     if (batch_pts > h->ptcap) {
         int64_t pc = h->ptcap * 2 > batch_pts ? h->ptcap * 2 : batch_pts;
-        CKH(h, join_metrics(h));   // they read the buffers replaced below
         if (pc < 4096) pc = 4096;
         if (pc >= ((int64_t)1 << 31) - 1) {
             h->err = "too many points in one batch";
@@ -709,22 +706,6 @@ static WorkBufs handle_bufs(gvom_handle *h) {
     return w;
 }
 
-// Captures a non-overlapped stage's metrics on `side`, after what is on the main stream now: they
-// read work buffers and write slot records only, and run beside the commit and the next
-// combine's table pass, which need neither (14 us for 12k voxels, latency-bound, beside a pass
-// bound by its reads).  Only inside a capture, where the dependencies become graph edges (8
-// frames of 131,072 points 963 -> 918 us a launch): eager calls pay for the events, a frame of
-// the same scans took 158 us instead of 150, 151 x 151 x 100 128 instead of 111.
-static int metrics_aside(gvom_handle *h, const WorkBufs &W, int64_t NT, int S) {
-    CKH(h, hipEventRecord(h->ev_front, h->stream));
-    CKH(h, hipStreamWaitEvent(h->side, h->ev_front, 0));
-    CKH(h, launch_metrics(W.seg_key, W.mom, NT, h->g, h->st, h->slot_tables, h->slot_recs, h->ncap, S, h->side));
-    CKH(h, hipEventRecord(h->ev_metrics, h->side));
-    h->metrics_pending = true;
-    h->metrics_on_side = true;
-    return GVOM_OK;
-}
-
 // The scan stage for S scans (gvom.py:105-220 for each).
 // cast = false (gvom_diff_forward in geometry-only mode): no ray cast; the slot tables are
 // cleared instead, so the slot holds the occupied voxels and records without pass counts.
@@ -840,10 +821,7 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     // a stage on the main stream reuses the work buffers pending metrics still read; an
     // overlapped one runs on `front` after them
     if (!ovl) CKH(h, join_metrics(h));
-    if (ovl) {
-        CKH(h, hipStreamWaitEvent(fs, h->ev_back, 0));
-        if (h->metrics_on_side) CKH(h, hipStreamWaitEvent(fs, h->ev_metrics, 0));
-    }
+    if (ovl) CKH(h, hipStreamWaitEvent(fs, h->ev_back, 0));
     const size_t esz = dtype == GVOM_F32 ? 4 : 8;
     const void *pts = xyz;
     ScanDesc *sd = h->sd;
@@ -941,16 +919,11 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
         CKH(h, hipEventRecord(h->ev_front, fs));
         CKH(h, hipStreamWaitEvent(st, h->ev_front, 0));
         h->metrics_pending = false;   // `front` ran any earlier stage's metrics before ev_front
-        CKH(h, launch_metrics(W.seg_key, W.mom, NT, g, h->st, h->slot_tables, h->slot_recs, h->ncap, S, fs));
+    }
+    CKH(h, launch_metrics(W.seg_key, W.mom, NT, g, h->st, h->slot_tables, h->slot_recs, h->ncap, S, fs));
+    if (ovl) {
         CKH(h, hipEventRecord(h->ev_metrics, fs));
         h->metrics_pending = true;
-        h->metrics_on_side = false;
-    } else if (h->capturing && !h->cap_sd_dev) {
-        const int rc_m = metrics_aside(h, W, NT, S);
-        if (rc_m) return rc_m;
-    } else {
-        // an eager call waits for an event of another stream longer than the metrics take
-        CKH(h, launch_metrics(W.seg_key, W.mom, NT, g, h->st, h->slot_tables, h->slot_recs, h->ncap, S, fs));
     }
     CKH(h, launch_commit_process(h->st, sd, g, S, st));
     stage_event(h, 4);
@@ -1947,7 +1920,6 @@ extern "C" int gvom_graph_begin(gvom_handle *h, int32_t max_scans) {
         ++h->buf_gen;
     }
     CKH(h, hipStreamSynchronize(h->stream));
-    h->metrics_on_side = false;   // joined above, and done
     h->cap_ops.clear();
     h->cap_sd.clear();
     h->mirror_next = h->next_slot;
@@ -1972,7 +1944,6 @@ extern "C" int gvom_graph_end(gvom_handle *h, gvom_graph **out) {
         return GVOM_ESTATE;
     }
     h->capturing = false;
-    h->metrics_on_side = false;   // the sequence's end follows its metrics
     // nothing ran: restore the host mirror; gvom_graph_launch replays the bookkeeping
     h->next_slot = h->mirror_next;
     h->last_slot = h->mirror_last;

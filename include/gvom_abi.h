@@ -10,9 +10,7 @@
  *   - entry points return 0 on success, GVOM_NO_DATA (1) where the reference returns
  *     None, and a negative GVOM_E* code on error; gvom_last_error() gives the text;
  *   - every call on one handle is serialised by a per-handle mutex, and all device
- *     work of a handle runs in order on one HIP stream, but for what no caller can see
- *     before the next call on the handle (a scan's neighbourhood metrics run beside
- *     its commit and the next combine's table pass, see gvom_set_overlap);
+ *     work of a handle runs in order on one HIP stream;
  *   - "_device" variants take device pointers and do not synchronise the stream.
  *
  * Map layout of all 2D outputs: C-order [x, y] arrays of xy_size * xy_size, as the
