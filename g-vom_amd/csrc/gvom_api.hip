@@ -112,7 +112,8 @@ struct gvom_handle {
     int device = 0;
     hipStream_t stream = nullptr;
     // second stream for the sort / segment / chunk-partial chain, which does not depend on
-    // the ray cast; forked after k_prepare and joined before the segment sums
+    // the ray cast; forked after k_prepare and joined before the segment sums where
+    // that pays (process_impl)
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     // caller-stream hand-off of the stream-ordered entry points: ev_in on the caller's stream,
@@ -878,15 +879,27 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
                           xcd ? RAY_SECTORS : (az ? RAY_AZIMUTH : RAY_LINEAR), W.rsec, W.hist, W.hwords, W.azhist,
                           W.azwords, fs));
     if (xcd) CKH(h, launch_ray_order(W.rsec, NT, h->st, W.rorder, fs));
-    // fork: keys, segments and chunk partials on the side stream, concurrent with the cast
-    CKH(h, hipEventRecord(h->ev_fork, fs));
-    CKH(h, hipStreamWaitEvent(h->side, h->ev_fork, 0));
+    // fork: keys, segments and chunk partials on the side stream, concurrent with the cast, where
+    // that saves more than the two events and their waits cost.  An eager call of a small scan
+    // stays on one stream: 46k points on 151 x 151 x 100 (tiled cast) take 111 us a frame with
+    // the fork and 89 without, the host's side 110 and 55 us.  From the azimuth cast's size on the
+    // fork pays (131,072 points on 256 x 256 x 64 164 us with it and 168 without, 212k on 512 x
+    // 512 x 64 372 and 409), and in a captured sequence, where the events are graph edges, at
+    // every size (a replayed host call, 7,763 points on 64 x 64 x 32, 114 and 119 us).  Without a
+    // cast only a table clear runs beside the chain, and one stream is faster in a replayed
+    // loss call as well (62k points on 256 x 256 x 64 338 and 307 us).
+    const bool fork = cast && (h->capturing || gvom_plan::az_pays(NT, g.XY));
+    hipStream_t cs = fork ? h->side : fs;
+    if (fork) {
+        CKH(h, hipEventRecord(h->ev_fork, fs));
+        CKH(h, hipStreamWaitEvent(cs, h->ev_fork, 0));
+    }
     uint32_t *sk = W.k0, *sv = W.v0;
-    CKH(h, radix_sort(W.k0, W.v0, W.k1, W.v1, NT, g.VB + sbits, g.VB, W.hist, W.hwords, h->st, &sk, &sv, h->side));
+    CKH(h, radix_sort(W.k0, W.v0, W.k1, W.v1, NT, g.VB + sbits, g.VB, W.hist, W.hwords, h->st, &sk, &sv, cs));
     h->sorted_vals = sv;
     CKH(h, launch_segments(dtype, W.world, sk, sv, NT, sd, S, g, h->st, W.hist, W.hwords, W.blk, W.blk_words,
-                           W.seg_start, W.seg_key, W.part, h->side));
-    CKH(h, hipEventRecord(h->ev_join, h->side));
+                           W.seg_start, W.seg_key, W.part, cs));
+    if (fork) CKH(h, hipEventRecord(h->ev_join, cs));
     // the tiled path's conversion writes every word of the slot tables; the direct casts count
     // into cleared tables, cleared here, beside the sort chain (nothing before the cast reads them)
     if (az)
@@ -908,7 +921,7 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
                                    h->slot_table_words, fs));
     stage_event(h, 2, fs);
     // join: the segment sums read the pass counts and the partials
-    CKH(h, hipStreamWaitEvent(fs, h->ev_join, 0));
+    if (fork) CKH(h, hipStreamWaitEvent(fs, h->ev_join, 0));
     stage_event(h, 3, fs);
     CKH(h, launch_mom_seg(W.seg_start, W.seg_key, NT, g, h->st, h->slot_tables, h->slot_recs, h->ncap, W.part,
                           W.mom, fs));
