@@ -263,8 +263,11 @@ struct gvom_handle {
     // `front`.  hipStreamEndCapture has crashed on that nested fork under an older HIP runtime
     // than the one this library is built against (torch bundles one, and when torch is imported
     // first this library binds to it: both have the SONAME libamdhip64.so.7).  Under an older
-    // runtime a captured sequence therefore runs its scan stages on the main stream, as with
-    // overlap off; eager calls still overlap.
+    // runtime a captured overlapped stage therefore runs whole on `side`, its sort chain before
+    // its cast, so that the sequence holds the main stream and one stream forked from it, as with
+    // overlap off: 8 frames of 131,072 points on 256 x 256 x 64 take 865 us a launch, with the
+    // stages on the main stream 955.  Under the newer runtime the nested fork is the faster form
+    // (the same frames 115 us each, 134 with the stage whole on `side`).
     int runtime_version = 0;
     bool nested_capture = true;
     int diff_geometry = 0;   // gvom_set_diff_geometry_only
@@ -817,8 +820,11 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     // (new_buf), never what a combine reads; with overlap on it runs on `front` and may proceed
     // while a combine enqueued before this call still runs on st.  Only its commit (ring
     // state, buffer bits) goes on st, after that combine.
-    const bool ovl = h->overlap && on_device && may_overlap && (h->nested_capture || !h->capturing);
-    hipStream_t fs = ovl ? h->front : st;
+    const bool ovl = h->overlap && on_device && may_overlap;
+    // inside a capture under an older HIP runtime the whole stage runs on `side`, the one stream
+    // forked from the main stream then (see nested_capture)
+    const bool flat = h->capturing && !h->nested_capture;
+    hipStream_t fs = !ovl ? st : flat ? h->side : h->front;
     // a stage on the main stream reuses the work buffers pending metrics still read; an
     // overlapped one runs on `front` after them
     if (!ovl) CKH(h, join_metrics(h));
@@ -888,7 +894,7 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     // every size (a replayed host call, 7,763 points on 64 x 64 x 32, 114 and 119 us).  Without a
     // cast only a table clear runs beside the chain, and one stream is faster in a replayed
     // loss call as well (62k points on 256 x 256 x 64 338 and 307 us).
-    const bool fork = cast && (h->capturing || gvom_plan::az_pays(NT, g.XY));
+    const bool fork = cast && !(ovl && flat) && (h->capturing || gvom_plan::az_pays(NT, g.XY));
     hipStream_t cs = fork ? h->side : fs;
     if (fork) {
         CKH(h, hipEventRecord(h->ev_fork, fs));
