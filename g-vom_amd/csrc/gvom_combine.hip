@@ -927,58 +927,55 @@ __global__ __launch_bounds__(256) void k_export_table(Geo g, const int32_t *__re
 __global__ __launch_bounds__(256) void k_debug_voxels(Geo g, const DevState *__restrict__ st, int par,
                                                       const int32_t *__restrict__ table,
                                                       const CombRec *__restrict__ recs,
-                                                      float *__restrict__ out) {
+                                                      float4 *__restrict__ out) {
     int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= g.V) return;
     int32_t t = table[v];
     if (t >= 0) return;
-    uint32_t id = (uint32_t)t & MASK31;
+    const int64_t id = (int64_t)((uint32_t)t & MASK31);
     int64_t z = v % g.Z, c = v / g.Z, y = c % g.XY, x = c / g.XY;
     const double *o = st->comb_origin[par];
     const CombRec &r = recs[id];
-    float *row = out + (int64_t)id * 8;
-    row[0] = (float)(((double)x + o[0]) * g.xy_res);
-    row[1] = (float)(((double)y + o[1]) * g.xy_res);
-    row[2] = (float)(((double)z + o[2]) * g.z_res);
-    row[3] = (float)((double)r.hit / (double)r.total);
-    row[4] = (float)r.hit;
-    row[5] = r.ev[0] - r.ev[1];
-    row[6] = r.ev[1] - r.ev[2];
-    row[7] = r.ev[2];
+    out[2 * id] = make_float4((float)(((double)x + o[0]) * g.xy_res), (float)(((double)y + o[1]) * g.xy_res),
+                               (float)(((double)z + o[2]) * g.z_res), (float)((double)r.hit / (double)r.total));
+    out[2 * id + 1] = make_float4((float)r.hit, r.ev[0] - r.ev[1], r.ev[1] - r.ev[2], r.ev[2]);
 }
 
-// __make_height_map_pointcloud (gvom.py:456-468) and __make_infered_height_map_pointcloud
-// (471-479, fed with the guessed height delta, 439-440); row index x + y*xy.
+// __make_height_map_pointcloud (gvom.py:456-468; W = 7), with the positive-obstacle map beside it
+// as the node's records have it (W = 8, gvom_ros.py:176-186), and
+// __make_infered_height_map_pointcloud (471-479, fed with the guessed height delta, 439-440; W =
+// 3): rows of W words, row index x + y*xy.  A block's 256 rows are put together in LDS and
+// written as one run of words.
+template <int W>
 __global__ __launch_bounds__(256) void k_debug_height(Geo g, const DevState *__restrict__ st, int par,
                                                       const double *__restrict__ height,
                                                       const double *__restrict__ rough,
                                                       const double *__restrict__ sx,
                                                       const double *__restrict__ sy,
                                                       const double *__restrict__ delta,
-                                                      float *__restrict__ out7, float *__restrict__ out3) {
-    int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= g.X) return;
-    int64_t x = c / g.XY, y = c % g.XY;
-    int64_t row = x + y * g.XY;
-    const double *o = st->comb_origin[par];
-    float fx = (float)(((double)x + o[0]) * g.xy_res);
-    float fy = (float)(((double)y + o[1]) * g.xy_res);
-    if (out7) {
-        float *r = out7 + row * 7;
-        r[0] = fx;
-        r[1] = fy;
-        r[2] = (float)(height[c] - g.z_res);
-        r[3] = (float)rough[c];
-        r[4] = (float)sx[c];
-        r[5] = (float)sy[c];
-        r[6] = (float)sqrt(sx[c] * sx[c] + sy[c] * sy[c]);
+                                                      const int32_t *__restrict__ pos,
+                                                      uint32_t *__restrict__ out) {
+    __shared__ uint32_t w[256 * W];
+    const int64_t base = (int64_t)blockIdx.x * 256, row = base + threadIdx.x;
+    if (row < g.X) {
+        const int64_t y = row / g.XY, x = row - y * g.XY, c = x * g.XY + y;
+        const double *o = st->comb_origin[par];
+        uint32_t *r = w + threadIdx.x * W;
+        r[0] = __float_as_uint((float)(((double)x + o[0]) * g.xy_res));
+        r[1] = __float_as_uint((float)(((double)y + o[1]) * g.xy_res));
+        r[2] = __float_as_uint((float)((W == 3 ? delta[c] : height[c]) - g.z_res));
+        if (W > 3) {
+            const double a = sx[c], b = sy[c];
+            r[3] = __float_as_uint((float)rough[c]);
+            r[4] = __float_as_uint((float)a);
+            r[5] = __float_as_uint((float)b);
+            r[6] = __float_as_uint((float)sqrt(a * a + b * b));
+            if (W == 8) r[7] = (uint32_t)pos[c];
+        }
     }
-    if (out3) {
-        float *r = out3 + row * 3;
-        r[0] = fx;
-        r[1] = fy;
-        r[2] = (float)(delta[c] - g.z_res);
-    }
+    __syncthreads();
+    const int64_t left = (g.X - base) * W, n = left < 256 * W ? left : 256 * W;
+    for (int64_t k = threadIdx.x; k < n; k += 256) out[base * W + k] = w[k];
 }
 
 inline unsigned nblocks(int64_t n, int per) { return (unsigned)((n + per - 1) / per > 0 ? (n + per - 1) / per : 1); }
@@ -1059,15 +1056,25 @@ hipError_t launch_export_table(const Geo &g, const int32_t *table, int32_t *out_
 }
 
 hipError_t launch_debug_voxels(const Geo &g, const DevState *st, const int32_t *comb_tables,
-                               const CombRec *comb_recs, int64_t ccap, int parity, float *out, hipStream_t s) {
+                               const CombRec *comb_recs, int64_t ccap, int parity, float *out,
+                               hipStream_t s) {
     k_debug_voxels<<<nblocks(g.V, 256), 256, 0, s>>>(g, st, parity, comb_tables + (int64_t)parity * g.V,
-                                                     comb_recs + (int64_t)parity * ccap, out);
+                                                     comb_recs + (int64_t)parity * ccap, (float4 *)out);
     return hipGetLastError();
 }
 
 hipError_t launch_debug_height(const Geo &g, const DevState *st, int parity, const double *height,
                                const double *rough, const double *sx, const double *sy, const double *delta,
-                               float *out7, float *out3, hipStream_t s) {
-    k_debug_height<<<nblocks(g.X, 256), 256, 0, s>>>(g, st, parity, height, rough, sx, sy, delta, out7, out3);
+                               const int32_t *pos, int width, float *out, hipStream_t s) {
+    const unsigned nb = nblocks(g.X, 256);
+    uint32_t *o = (uint32_t *)out;
+    if (width == 3)
+        k_debug_height<3><<<nb, 256, 0, s>>>(g, st, parity, height, rough, sx, sy, delta, pos, o);
+    else if (width == 7)
+        k_debug_height<7><<<nb, 256, 0, s>>>(g, st, parity, height, rough, sx, sy, delta, pos, o);
+    else if (width == 8)
+        k_debug_height<8><<<nb, 256, 0, s>>>(g, st, parity, height, rough, sx, sy, delta, pos, o);
+    else
+        return hipErrorInvalidValue;
     return hipGetLastError();
 }

@@ -6,6 +6,8 @@
 
 // ---- fills --------------------------------------------------------------------------
 hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t s);
+// bytes from device memory to pinned host memory, both 16-byte aligned
+hipError_t launch_copy(void *dst, const void *src, int64_t bytes, hipStream_t s);
 
 // ---- scan stage (gvom_scan.hip) ------------------------------------------------------
 // Transform, validity, own-voxel sort key per point (reference gvom.py:1122-1163).
@@ -118,7 +120,8 @@ hipError_t launch_debug_voxels(const Geo &g, const DevState *st, const int32_t *
                                hipStream_t s);
 hipError_t launch_debug_height(const Geo &g, const DevState *st, int parity, const double *height,
                                const double *rough, const double *sx, const double *sy,
-                               const double *delta, float *out7, float *out3, hipStream_t s);
+                               const double *delta, const int32_t *pos, int width, float *out,
+                               hipStream_t s);
 
 
 // ---- image kernels the reference defines but never calls (gvom_image.hip) -------------------

@@ -304,20 +304,32 @@ class Gvom:
         if rc == nat.GVOM_NO_DATA:
             print("No data")
             return None
-        out = np.zeros((rows.value, 8), np.float32)
+        out = np.empty((rows.value, 8), np.float32)
         nat.check(self._lib.gvom_debug_voxel_map(self._h, nat.ptr(out), rows.value, ctypes.byref(rows)), self._h)
         return out
 
     def make_debug_height_map(self):
-        out = np.zeros((self.xy_size * self.xy_size, 7), np.float32)
+        out = np.empty((self.xy_size * self.xy_size, 7), np.float32)
         rc = nat.check(self._lib.gvom_debug_height_map(self._h, nat.ptr(out)), self._h)
         if rc == nat.GVOM_NO_DATA:
             print("No data")
             return None
         return out
 
+    def height_map_records(self, dtype):
+        """The node's height-map records: make_debug_height_map's columns and the positive obstacle
+        map (int32) in a structured array of `dtype` (eight 4-byte fields)."""
+        out = np.empty(self.xy_size * self.xy_size, dtype)
+        if out.dtype.itemsize != 32:
+            raise ValueError("records of eight 4-byte fields expected")
+        rc = nat.check(self._lib.gvom_debug_height_records(self._h, nat.ptr(out)), self._h)
+        if rc == nat.GVOM_NO_DATA:
+            print("No data")
+            return None
+        return out
+
     def make_debug_inferred_height_map(self):
-        out = np.zeros((self.xy_size * self.xy_size, 3), np.float32)
+        out = np.empty((self.xy_size * self.xy_size, 3), np.float32)
         rc = nat.check(self._lib.gvom_debug_inferred_height_map(self._h, nat.ptr(out)), self._h)
         if rc == nat.GVOM_NO_DATA:
             print("No data")

@@ -41,6 +41,7 @@ SIGNATURES = {
     "gvom_occupancy_grids": (ctypes.c_int, [_P, ctypes.c_double, ctypes.c_double, ctypes.c_double, _P, _I32, _P]),
     "gvom_debug_voxel_map": (ctypes.c_int, [_P, _P, _I64, _P]),
     "gvom_debug_height_map": (ctypes.c_int, [_P, _P]),
+    "gvom_debug_height_records": (ctypes.c_int, [_P, _P]),
     "gvom_debug_inferred_height_map": (ctypes.c_int, [_P, _P]),
     "gvom_get_slot": (ctypes.c_int, [_P, _I32, _P, _I64, _P, _P, _P, _P, _P, _P]),
     "gvom_get_combined": (ctypes.c_int, [_P, _P, _I64, _P, _P, _P, _P, _P, _P, _P]),

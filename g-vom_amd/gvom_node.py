@@ -69,6 +69,22 @@ def _position(odom):
     return (float(x), float(y), float(z))
 
 
+def _record(names, last="f4"):
+    names = names.split(",")
+    return np.dtype([(n, "f4") for n in names[:-1]] + [(names[-1], last)])
+
+
+# The debug clouds' rows; the arrays the mapper returns hold them as they are.
+VOXEL_RECORD = _record("x,y,z,solid factor,count,eigen_line,eigen_surface,eigen_point")
+HEIGHT_RECORD = _record("x,y,z,roughness,slope_x,slope_y,slope,obstacles", "i4")
+INFERRED_RECORD = _record("x,y,z")
+
+
+def _records(rows, dtype):
+    """Float32 rows as a record array over the same memory."""
+    return rows.reshape(-1).view(dtype).view(np.recarray)
+
+
 @dataclass
 class GridInfo:
     """nav_msgs/MapMetaData as the node fills it (gvom_ros.py:124-135)."""
@@ -151,14 +167,11 @@ class GvomNode:
         out = {}
         v = m.make_debug_voxel_map()
         if v is not None:
-            out["voxel"] = np.rec.fromarrays([v[:, k] for k in range(8)],
-                                             names="x,y,z,solid factor,count,eigen_line,eigen_surface,eigen_point")
-        h = m.make_debug_height_map()
+            out["voxel"] = _records(v, VOXEL_RECORD)
+        h = m.height_map_records(HEIGHT_RECORD)
         if h is not None:
-            obs = m.maps_state()["pos"]
-            out["height_map"] = np.rec.fromarrays([h[:, k] for k in range(7)] + [obs.flatten("F")],
-                                                  names="x,y,z,roughness,slope_x,slope_y,slope,obstacles")
+            out["height_map"] = h.view(np.recarray)
         i = m.make_debug_inferred_height_map()
         if i is not None:
-            out["inferred_height_map"] = np.rec.fromarrays([i[:, k] for k in range(3)], names="x,y,z")
+            out["inferred_height_map"] = _records(i, INFERRED_RECORD)
         return out

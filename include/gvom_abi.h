@@ -213,6 +213,10 @@ int gvom_debug_voxel_map(gvom_handle *h, float *out, int64_t cap, int64_t *rows)
 /* Replaces Gvom.make_debug_height_map (gvom.py:411-425): xy_size^2 rows of 7 floats. */
 int gvom_debug_height_map(gvom_handle *h, float *out);
 
+/* The node's height-map records (gvom_ros.py:176-186): the same rows with the positive
+ * obstacle map (int32) as an eighth word, xy_size^2 rows of 32 bytes. */
+int gvom_debug_height_records(gvom_handle *h, void *out);
+
 /* Replaces Gvom.make_debug_inferred_height_map (gvom.py:427-442): xy_size^2 rows of 3. */
 int gvom_debug_inferred_height_map(gvom_handle *h, float *out);
 
