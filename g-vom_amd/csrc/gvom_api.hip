@@ -876,7 +876,7 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
             h->pin_next = 1 - k;
             pts = W.pts_in;
         }
-        CKH(h, hipMemcpyAsync(h->sd, sdh, sizeof(ScanDesc) * S, hipMemcpyHostToDevice, fs));
+        CKH(h, launch_set_descs(h->sd, sdh, S, fs));
     }
     h->diff_n = -1;   // every check passed: the work buffers a pending gvom_diff_backward reads are reused below
     stage_event(h, 0, fs);
@@ -944,12 +944,13 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
         CKH(h, hipStreamWaitEvent(st, h->ev_front, 0));
         h->metrics_pending = false;   // `front` ran any earlier stage's metrics before ev_front
     }
-    CKH(h, launch_metrics(W.seg_key, W.mom, NT, g, h->st, h->slot_tables, h->slot_recs, h->ncap, S, fs));
+    CKH(h, launch_metrics(W.seg_key, W.mom, NT, g, h->st, h->slot_tables, h->slot_recs, h->ncap, S,
+                          ovl ? nullptr : sd, fs));
     if (ovl) {
         CKH(h, hipEventRecord(h->ev_metrics, fs));
         h->metrics_pending = true;
+        CKH(h, launch_commit_process(h->st, sd, g, S, st));
     }
-    CKH(h, launch_commit_process(h->st, sd, g, S, st));
     stage_event(h, 4);
     CKH(h, mark_back(h));
 

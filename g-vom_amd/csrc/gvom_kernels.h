@@ -16,6 +16,7 @@ hipError_t launch_copy(void *dst, const void *src, int64_t bytes, hipStream_t s)
 // counted in st) or RAY_AZIMUTH (azimuth bins, counted in azhist, azwords words, which must be
 // zero).
 enum RayMode { RAY_LINEAR = 0, RAY_SECTORS = 1, RAY_AZIMUTH = 2 };
+hipError_t launch_set_descs(ScanDesc *sd, const ScanDesc *host, int S, hipStream_t s);
 hipError_t launch_prepare(int dtype, const void *in, void *world, uint32_t *keys, uint32_t *vals,
                           uint8_t *valid, const ScanDesc *sd, int S, int64_t NT, const Geo &g,
                           DevState *st, int rmode, uint8_t *rbin, uint32_t *hist, int64_t hwords, uint32_t *azhist,
@@ -76,7 +77,7 @@ hipError_t launch_mom_seg(const int32_t *seg_start, const uint32_t *seg_key, int
 // Neighbourhood mean/covariance per occupied voxel (gvom.py:1250-1387).
 hipError_t launch_metrics(const uint32_t *seg_key, const Moment *mom, int64_t seg_cap, const Geo &g,
                           DevState *st, const int32_t *slot_tables, SlotRec *slot_recs, int64_t ncap, int S,
-                          hipStream_t s);
+                          const ScanDesc *commit_sd, hipStream_t s);
 // One-wave commit of the S scans: slot origins, latest ego, buffer bits, cell counts, ring
 // indices and the next combine's source shifts.
 hipError_t launch_commit_process(DevState *st, const ScanDesc *sd, const Geo &g, int S, hipStream_t s);

