@@ -1867,13 +1867,14 @@ __global__ __launch_bounds__(256) void k_copy(uint8_t *__restrict__ dst, const u
 // from pageable memory costs the host a staging copy and the stream a copy kernel.  With the commit
 // as a block of the metrics and ten lanes storing a record's ten values, a frame of 46k points on
 // 151 x 151 x 100 went from 88.6 to 86.3 us, one of 131,072 on 256 x 256 x 64 from 147.8 to 145.1.
-constexpr int DESC_ARGS = 4;
-struct DescArgs {
-    ScanDesc d[DESC_ARGS];
+// N = 16 (2.3 of the 4 KB a launch's arguments may take) keeps the largest batch at two launches.
+template <int N> struct DescArgs {
+    ScanDesc d[N];
 };
 static_assert(sizeof(ScanDesc) % 4 == 0 && sizeof(ScanDesc) / 4 <= 64, "a lane per word of a descriptor");
 
-__global__ __launch_bounds__(64 * DESC_ARGS) void k_set_descs(ScanDesc *__restrict__ sd, DescArgs a, int n) {
+template <int N>
+__global__ __launch_bounds__(64 * N) void k_set_descs(ScanDesc *__restrict__ sd, DescArgs<N> a, int n) {
     const int s = threadIdx.x >> 6, w = threadIdx.x & 63;
     if (s < n && w < (int)(sizeof(ScanDesc) / 4))
         reinterpret_cast<uint32_t *>(sd + s)[w] = reinterpret_cast<const uint32_t *>(a.d + s)[w];
@@ -1902,14 +1903,19 @@ hipError_t launch_copy(void *dst, const void *src, int64_t bytes, hipStream_t s)
     return hipGetLastError();
 }
 
+template <int N> static void set_descs(ScanDesc *sd, const ScanDesc *host, int n, hipStream_t s) {
+    DescArgs<N> a;
+    std::memset((void *)&a, 0, sizeof(a));
+    std::memcpy((void *)a.d, host, sizeof(ScanDesc) * n);
+    k_set_descs<N><<<1, 64 * N, 0, s>>>(sd, a, n);
+}
+
 hipError_t launch_set_descs(ScanDesc *sd, const ScanDesc *host, int S, hipStream_t s) {
     if (S < 1 || S > GVOM_MAX_BATCH) return hipErrorInvalidValue;
-    for (int at = 0; at < S; at += DESC_ARGS) {
-        DescArgs a;
-        const int n = S - at < DESC_ARGS ? S - at : DESC_ARGS;
-        std::memset((void *)&a, 0, sizeof(a));
-        std::memcpy((void *)a.d, host + at, sizeof(ScanDesc) * n);
-        k_set_descs<<<1, 64 * DESC_ARGS, 0, s>>>(sd + at, a, n);
+    if (S <= 2) {
+        set_descs<2>(sd, host, S, s);
+    } else {
+        for (int at = 0; at < S; at += 16) set_descs<16>(sd + at, host + at, S - at < 16 ? S - at : 16, s);
     }
     return hipGetLastError();
 }
