@@ -1631,7 +1631,8 @@ __device__ __forceinline__ int64_t neighbour_segment(int64_t x, int64_t y, int64
 // (swapped neighbours, swapped pairs, mirrored halves, mirrored rows: after each step the
 // lanes that were summed hold the same value, so a mirror acts as the next power of two), and
 // only the last step goes through the LDS crossbar, which a shuffle of every step filled (ten
-// f64 sums per voxel): k_metrics 16.2 -> 14.1 us for 12k voxels, 38 -> 31 for 40k.
+// f64 sums per voxel): k_metrics 16.2 -> 14.1 us for 12k voxels, 38 -> 31 for 40k (13.4 and 29 since ten
+// lanes store a record).
 template <int CTRL> __device__ __forceinline__ double dpp_add(double v) {
     const int lo = __double2loint(v), hi = __double2hiint(v);
     return v + __hiloint2double(__builtin_amdgcn_mov_dpp(hi, CTRL, 0xF, 0xF, false),
