@@ -911,17 +911,22 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
         CKH(h, hipStreamWaitEvent(cs, h->ev_fork, 0));
     }
     uint32_t *sk = W.k0, *sv = W.v0;
-    CKH(h, radix_sort(W.k0, W.v0, W.k1, W.v1, NT, g.VB + sbits, g.VB, W.hist, W.hwords, h->st, &sk, &sv, cs));
+    // the direct casts count into cleared tables; on one stream the sort's first pass, which leaves
+    // most of the chip idle, clears them
+    const bool own_clear = !az && !tiled && (fork || NT <= 0);
+    const SlotClear clear{h->slot_tables, g.B, S, g.V};
+    CKH(h, radix_sort(W.k0, W.v0, W.k1, W.v1, NT, g.VB + sbits, g.VB, W.hist, W.hwords, h->st, &sk, &sv, cs,
+                      !az && !tiled && !own_clear ? &clear : nullptr));
     h->sorted_vals = sv;
     CKH(h, launch_segments(dtype, W.world, sk, sv, NT, sd, S, g, h->st, W.hist, W.hwords, W.blk, W.blk_words,
                            W.seg_start, W.seg_key, W.part, cs));
     if (fork) CKH(h, hipEventRecord(h->ev_join, cs));
-    // the tiled path's conversion writes every word of the slot tables; the direct casts count
-    // into cleared tables, cleared here, beside the sort chain (nothing before the cast reads them)
+    // the tiled path's conversion writes every word of the slot tables; beside a forked sort chain
+    // the direct casts' tables are cleared here (nothing before the cast reads them)
     if (az)
         CKH(h, launch_az_order(W.rsec, W.valid, sd, S, NT, g, h->st, W.azhist, W.azwords, W.rorder, h->slot_tables,
                                h->slot_table_words, -1, fs));
-    else if (!tiled) CKH(h, launch_clear_slots(h->slot_tables, h->st, S, g, fs));
+    else if (own_clear) CKH(h, launch_clear_slots(h->slot_tables, h->st, S, g, fs));
     stage_event(h, 1, fs);
     if (az)
         CKH(h, launch_raycast_az(dtype, W.world, sd, S, NT, g, h->st, h->slot_tables, h->slot_table_words, W.rorder,

@@ -55,9 +55,16 @@ hipError_t launch_raycast(int dtype, const void *world, const uint8_t *valid, co
 // buffer pair holds the result.
 // scan_shift: keys >> scan_shift is the scan of the batch (the first pass counts each scan's
 // valid keys into set 1).
+// The S slot tables of V words a scan stage counts into, cleared by the first pass of its sort.
+struct SlotClear {
+    int32_t *tables;
+    int B, S;
+    int64_t V;
+};
 hipError_t radix_sort(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, int64_t n, int bits, int scan_shift,
                       uint32_t *hist, int64_t hwords, DevState *st, uint32_t **kout, uint32_t **vout,
-                      hipStream_t s);
+                      hipStream_t s,
+                      const SlotClear *clear = nullptr);
 int64_t radix_hist_entries(int64_t n);
 // words of the segment kernels' per-block counts (launch_segments' blk) for n sorted keys
 int64_t segment_block_words(int64_t n);

@@ -1012,15 +1012,40 @@ __device__ __forceinline__ void rs_scatter_tile(uint32_t *__restrict__ kout, uin
     }
 }
 
+// Block cb of a launch's clear of its stage's target slot tables (clear_blocks per table),
+// RS_THREADS x 16 words.
+constexpr int CLEAR_WORDS = RS_THREADS * 16;
+
+__device__ __forceinline__ void clear_slots_block(int cb, int clear_blocks, int force_slot,
+                                                  int32_t *__restrict__ tables, const DevState *__restrict__ st, int B,
+                                                  int32_t V) {
+    const int s = cb / clear_blocks;
+    const int buf =
+        force_slot >= 0 ? force_slot : __builtin_amdgcn_readfirstlane(new_buf(st->flip, (st->next_slot + s) % B));
+    int32_t *t = tables + (int64_t)buf * V;
+    const int64_t base = (int64_t)(cb - s * clear_blocks) * CLEAR_WORDS;
+    if ((V & 3) == 0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int64_t j = base + (k * RS_THREADS + (int)threadIdx.x) * 4;
+            if (j < V) *reinterpret_cast<int4 *>(t + j) = make_int4(0, 0, 0, 0);
+        }
+    } else {
+        for (int k = 0; k < 16; ++k) {
+            const int64_t j = base + k * RS_THREADS + (int)threadIdx.x;
+            if (j < V) t[j] = 0;
+        }
+    }
+}
+
 // First pass.  hist: its per-tile digit counts (block-major, from k_prepare).  tot_next
 // (zero on entry, or null in a one-pass sort): the next digit's totals, accumulated here.
 // scan_cnt (zero on entry): valid keys (!= GVOM_NOKEY) per scan, the scan being key >> VB.
-__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint32_t *__restrict__ kin,
-                                                           const uint32_t *__restrict__ vin,
-                                                           uint32_t *__restrict__ kout, uint32_t *__restrict__ vout,
-                                                           int64_t n, int shift, const uint32_t *__restrict__ hist,
-                                                           int nblk, uint32_t *__restrict__ tot_next, int VB,
-                                                           uint32_t *__restrict__ scan_cnt) {
+__device__ __forceinline__ void rs_scatter_first(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                 uint32_t *__restrict__ kout, uint32_t *__restrict__ vout, int64_t n,
+                                                 int shift, const uint32_t *__restrict__ hist, int nblk,
+                                                 uint32_t *__restrict__ tot_next, int VB,
+                                                 uint32_t *__restrict__ scan_cnt) {
     __shared__ uint32_t wcnt[RS_WAVES][256];
     __shared__ uint32_t ptot[4][256], pbef[4][256];
     __shared__ uint32_t gbase[256], nh[256];
@@ -1082,11 +1107,18 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint32_t *__res
     rs_scatter_tile(kout, vout, n, shift, base, lane, w, wcnt, gbase, kk, vv, lo);
 }
 
+__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint32_t *__restrict__ kin,
+                                                           const uint32_t *__restrict__ vin,
+                                                           uint32_t *__restrict__ kout, uint32_t *__restrict__ vout,
+                                                           int64_t n, int shift, const uint32_t *__restrict__ hist,
+                                                           int nblk, uint32_t *__restrict__ tot_next, int VB,
+                                                           uint32_t *__restrict__ scan_cnt) {
+    rs_scatter_first(kin, vin, kout, vout, n, shift, hist, nblk, tot_next, VB, scan_cnt);
+}
+
 // The azimuth order: per scan, a stable scatter of the valid rays' indices by azimuth bin, as
 // the sort's first pass (hist: bin counts per row from k_prepare), by one block per row b < nblk
 // (the points of one scan in one tile, see az_rows); the blocks after them clear the S target slot tables, RS_THREADS x 16 words each, which the cast counts into.
-constexpr int CLEAR_WORDS = RS_THREADS * 16;
-
 __global__ __launch_bounds__(RS_THREADS) void k_az_order(const uint8_t *__restrict__ rbin,
                                                          const uint8_t *__restrict__ valid,
                                                          const ScanDesc *__restrict__ sd, int S, int nblk,
@@ -1099,23 +1131,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_az_order(const uint8_t *__restri
     __shared__ uint32_t gbase[256];
     __shared__ uint32_t wtot[4];
     if ((int)blockIdx.x >= nblk) {
-        const int cb = (int)blockIdx.x - nblk, s = cb / clear_blocks;
-        const int buf =
-            force_slot >= 0 ? force_slot : __builtin_amdgcn_readfirstlane(new_buf(st->flip, (st->next_slot + s) % B));
-        int32_t *t = tables + (int64_t)buf * V;
-        const int64_t base = (int64_t)(cb - s * clear_blocks) * CLEAR_WORDS;
-        if ((V & 3) == 0) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int64_t j = base + (k * RS_THREADS + (int)threadIdx.x) * 4;
-                if (j < V) *reinterpret_cast<int4 *>(t + j) = make_int4(0, 0, 0, 0);
-            }
-        } else {
-            for (int k = 0; k < 16; ++k) {
-                const int64_t j = base + k * RS_THREADS + (int)threadIdx.x;
-                if (j < V) t[j] = 0;
-            }
-        }
+        clear_slots_block((int)blockIdx.x - nblk, clear_blocks, force_slot, tables, st, B, V);
         return;
     }
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1850,6 +1866,23 @@ __global__ __launch_bounds__(256) void k_fill_i32(int32_t *__restrict__ p, int32
     }
 }
 
+// The sort's first pass with the clear of the stage's target slot tables by the blocks from nblk on:
+// the pass has a block per 2048 keys, so the clear of 16 MiB runs on compute units it leaves idle
+// instead of in a launch of its own (8 captured frames of 131,072 points on one stream 860 -> 849
+// us).  A kernel beside k_rs_scatter, for stages that clear nothing or elsewhere: with the branch
+// in it a frame of 46k points took 0.2 to 0.6 us longer.
+__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter_clear(
+    const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin, uint32_t *__restrict__ kout,
+    uint32_t *__restrict__ vout, int64_t n, const uint32_t *__restrict__ hist, int nblk,
+    uint32_t *__restrict__ tot_next, int VB, uint32_t *__restrict__ scan_cnt, int32_t *__restrict__ tables,
+    const DevState *__restrict__ st, int B, int32_t V, int clear_blocks) {
+    if ((int)blockIdx.x >= nblk) {
+        clear_slots_block((int)blockIdx.x - nblk, clear_blocks, -1, tables, st, B, V);
+        return;
+    }
+    rs_scatter_first(kin, vin, kout, vout, n, 0, hist, nblk, tot_next, VB, scan_cnt);
+}
+
 // Device memory to pinned host memory in 16-byte words, in order on the stream (a copy engine's
 // transfer adds a hand-over to and from it).  Bound by the bus: 1.3 MB take 25 us (52 GB/s) from
 // any grid of 16 blocks or more, 33 as an asynchronous copy.
@@ -2076,7 +2109,8 @@ int64_t radix_hist_entries(int64_t n) { return gvom_plan::radix_hist_words(n); }
 int64_t segment_block_words(int64_t n) { return gvom_plan::segment_block_words(n); }
 
 hipError_t radix_sort(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, int64_t n, int bits, int scan_shift,
-                      uint32_t *hist, int64_t hwords, DevState *st, uint32_t **kout, uint32_t **vout, hipStream_t s) {
+                      uint32_t *hist, int64_t hwords, DevState *st, uint32_t **kout, uint32_t **vout, hipStream_t s,
+                      const SlotClear *clear) {
     *kout = k0;
     *vout = v0;
     if (n <= 0) return hipSuccess;
@@ -2091,8 +2125,15 @@ hipError_t radix_sort(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, in
     for (int p = 0; p < passes; ++p) {
         uint32_t *tn = p + 1 < passes ? totals(p + 1) : nullptr;
         if (p == 0) {
-            k_rs_scatter<<<nblk, RS_THREADS, 0, s>>>(ka, va, kb, vb, n, 0, hist, nblk, tn, scan_shift,
-                                                      hist + hwords + gvom_plan::radix_scan_counts_at(n));
+            uint32_t *scan_cnt = hist + hwords + gvom_plan::radix_scan_counts_at(n);
+            if (clear) {
+                const int cb = (int)nblocks(clear->V, CLEAR_WORDS);
+                k_rs_scatter_clear<<<nblk + cb * clear->S, RS_THREADS, 0, s>>>(
+                    ka, va, kb, vb, n, hist, nblk, tn, scan_shift, scan_cnt, clear->tables, st, clear->B,
+                    (int32_t)clear->V, cb);
+            } else {
+                k_rs_scatter<<<nblk, RS_THREADS, 0, s>>>(ka, va, kb, vb, n, 0, hist, nblk, tn, scan_shift, scan_cnt);
+            }
             if (passes == 1) {
                 hipError_t e = launch_fill_i32((int32_t *)hist, 0, hwords, s);
                 if (e != hipSuccess) return e;

@@ -66,3 +66,34 @@ def test_streams_match_synchronised_frames(n):
         _same(ref, eager, f"eager {r}")
         _same(ref, over, f"overlap {r}")
         _same(ref, cap, f"captured {r}")
+
+
+# words per table: below, at and above a clearing block's 16384, and not a multiple of four
+@pytest.mark.parametrize("xy,z", [(8, 4), (32, 16), (37, 13), (64, 33)])
+@pytest.mark.parametrize("scans", [1, 3])
+def test_tables_cleared_by_the_sort(xy, z, scans):
+    """A direct cast on one stream counts into tables its sort's first pass clears: after frames that
+    used every buffer of every slot, the slots equal those of the tiled cast, which writes whole
+    tables; an empty scan, which has no sort, leaves an empty slot."""
+    import gvom
+    import gvom_native as nat
+    base = synth.workload(2).map_args
+    direct, tiled = (gvom.Gvom(*base[:2], xy, z, 3, *base[5:]) for _ in range(2))
+    direct.set_raycast_config(256, 1, False, False, False, False)
+    rng = np.random.default_rng(xy)
+    reach = 0.25 * xy * base[0]
+    for k in range(5):
+        n = 0 if k == 4 else 3000 + 100 * k
+        p = np.stack([rng.normal(0, reach, n), rng.normal(0, reach, n), rng.normal(-0.5, 0.4, n)], 1)
+        p = p.astype(np.float32)
+        dev = nat.DeviceArray(p if n else np.zeros((1, 3), np.float32))
+        off = np.linspace(0, n, scans + 1).astype(np.int64)
+        egos = np.array([[0.5 * k + 0.1 * s, -0.3 * k, 0.1] for s in range(scans)])
+        for g in (direct, tiled):
+            g.process_batch_device(dev, off, egos, None)
+            g.sync()
+    for s in range(3):
+        a, b = direct.slot_state(s), tiled.slot_state(s)
+        assert (a is None) == (b is None)
+        for key in a or ():
+            assert np.array_equal(a[key], b[key]), (s, key)
