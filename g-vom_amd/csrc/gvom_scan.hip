@@ -1643,25 +1643,23 @@ __device__ __forceinline__ int64_t neighbour_segment(int64_t x, int64_t y, int64
 }
 
 // 32 lanes (half a wavefront) per occupied voxel, one lane per neighbour; sums over
-// neighbours are reductions in a fixed lane order.  Within 16 lanes they move through DPP
-// (swapped neighbours, swapped pairs, mirrored halves, mirrored rows: after each step the
-// lanes that were summed hold the same value, so a mirror acts as the next power of two), and
-// only the last step goes through the LDS crossbar, which a shuffle of every step filled (ten
-// f64 sums per voxel): k_metrics 16.2 -> 14.1 us for 12k voxels, 38 -> 31 for 40k (13.4 and 29 since ten
-// lanes store a record).
+// neighbours are tree reductions in a fixed lane order, partners 16, 8, 4, 2 and 1 lanes apart.
+// Only the first step goes through the LDS crossbar, the others through DPP; a shuffle of every
+// step filled the crossbar (ten f64 sums per voxel): k_metrics 16.2 -> 14.1 us for 12k voxels, 38 ->
+// 31 for 40k (13.4 and 29 since ten lanes store a record).
 template <int CTRL> __device__ __forceinline__ double dpp_add(double v) {
     const int lo = __double2loint(v), hi = __double2hiint(v);
     return v + __hiloint2double(__builtin_amdgcn_mov_dpp(hi, CTRL, 0xF, 0xF, false),
                                 __builtin_amdgcn_mov_dpp(lo, CTRL, 0xF, 0xF, false));
 }
 __device__ __forceinline__ double red32(double v) {
-    v = dpp_add<0xB1>(v);    // quad_perm [1, 0, 3, 2]
-    v = dpp_add<0x4E>(v);    // quad_perm [2, 3, 0, 1]
-    v = dpp_add<0x141>(v);   // row_half_mirror
-    v = dpp_add<0x140>(v);   // row_mirror
     constexpr int XOR16 = 0x401F;
-    return v + __hiloint2double(__builtin_amdgcn_ds_swizzle(__double2hiint(v), XOR16),
-                                __builtin_amdgcn_ds_swizzle(__double2loint(v), XOR16));
+    v += __hiloint2double(__builtin_amdgcn_ds_swizzle(__double2hiint(v), XOR16),
+                          __builtin_amdgcn_ds_swizzle(__double2loint(v), XOR16));
+    v = dpp_add<0x128>(v);    // row_ror 8: lane ^ 8
+    v = dpp_add<0x124>(v);    // row_ror 4: lane ^ 4, as the values now repeat every 8 lanes
+    v = dpp_add<0x4E>(v);     // quad_perm [2, 3, 0, 1]: lane ^ 2
+    return dpp_add<0xB1>(v);  // quad_perm [1, 0, 3, 2]: lane ^ 1
 }
 
 // Ring bookkeeping after the scan stage of S scans (gvom.py:211-216): slot origins for
