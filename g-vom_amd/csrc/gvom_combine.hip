@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void k_comb_tables(Geo g, const DevState *__re
                                                      int32_t *__restrict__ col_count,
                                                      int32_t *__restrict__ group, uint64_t *__restrict__ occ_bits,
                                                      double *__restrict__ height, double *__restrict__ inferred,
-                                                     int zl, int cpw) {
+                                                     int zl, int cpw, int wave_groups) {
     // per wavefront: a byte of occupied and a byte of free bits (passes, no hit) per lane, as
     // 64-bit words of its columns
     __shared__ __align__(16) uint8_t occ_b[4][512], free_b[4][512];
@@ -212,8 +212,12 @@ __global__ __launch_bounds__(256) void k_comb_tables(Geo g, const DevState *__re
             height[cc] = h;
         }
     }
-    // the block's occupied voxels
+    // the occupied voxels of the wavefront's or the block's columns
     for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off);
+    if (wave_groups) {
+        if (lane == 0 && c0 < X) group[blockIdx.x * 4 + wv] = (int32_t)cnt;
+        return;
+    }
     if (lane == 0) wave_cells[wv] = cnt;
     __syncthreads();
     if (threadIdx.x == 0)
@@ -436,123 +440,146 @@ __device__ __forceinline__ void merge_cell(const Geo &g, const DevState *__restr
     eigen3(cm, out.ev);
 }
 
-// Cells of CELL_PARTS x 64 columns per block: ids in z order from each part's first id (the
-// occupied voxels of all columns before it), the table entry becomes OCC | id, and the record
-// merge of the cell: sources in slot order, then the previous combined map (gvom.py:280-298).
-// A thread finds its cell from the columns' occupancy words (prefix of their counts, then the
-// k-th bit), so no list of cells goes through memory.  The parts lie a CELL_PARTS-th of the map
-// apart: the cells crowd around the sensor, and a block of neighbouring columns there would
-// set the time.  The thread holding a column's lowest occupied voxel writes its height
-// (min_h + z + oz) * z_res (gvom.py:572-576).
+// Cells of the combined map, an equal share per thread whatever columns they are in: ids in z order
+// from the first column on, the table entry becomes OCC | id, and the record merge of the cell:
+// sources in slot order, then the previous combined map (gvom.py:280-298).  A block makes the
+// first id of every group of gcols columns from the table pass's counts (a prefix sum in LDS);
+// a thread finds its id's group there, the column from the group's column counts and the height
+// from the column's occupancy words, so no list of cells goes through memory.  The thread holding
+// a column's lowest occupied voxel writes its height (min_h + z + oz) * z_res (gvom.py:572-576).
 //
-// The first id: the block adds the table pass's counts of occupied voxels per group of gcols
-// columns (four per load, several loads in flight: one after another they set the time).
+// The ids are dealt out evenly because cells crowd: a wall fills whole columns, and with the cells
+// of 256 fixed columns to a block the fullest block set the time.  71k cells of a scene with walls
+// on 256 x 256 x 64 took 71 us that way and take 20.0 (8 slots), 204 and 48 with 30 slots, 98 and
+// 26 on 256 x 256 x 256 (85k cells); an even scene's 38k cells 16.3 and 16.9, 64 x 64 x 32 9.0 and
+// 9.4 (the column's counts are one more load in the chain).
 //
-// Bound by latency: a cell is a chain of table word -> source words -> records, twice for eight
-// slots, and the merges between them.  256 x 256 x 64, 8 slots, 38k cells: 16.6 us, where the
-// column scan, the ids with their list and the merge of the list took 4.7 + 5.3 + 14.5.
-constexpr int CELL_PARTS = 4;          // groups of 64 columns per block
-constexpr int CELL_THREADS = 256;
+// Bound by latency: a cell is a chain of column counts -> occupancy word -> table word -> source
+// words -> records, the last two twice for eight slots, and the merges between them.  Two
+// wavefronts fit a SIMD; one block of eight a compute unit gives every SIMD two and makes the
+// prefix sum once there.  512 blocks of four took 20.7 and 19.2 us on the 71k and 38k cells
+// above, 1024 30.5 and 19.0, 256 blocks of four 30.5 and 18.2.
+constexpr int CELL_THREADS = 512;
+constexpr int CELL_SCAN = 4;      // prefix sum: up to CELL_SCAN x 4 groups per thread
+constexpr int CELL_LOADS = 4;     // 16 in flight: 0.4 to 0.9 us longer
+constexpr int CELL_BLOCKS = 256;
+constexpr int CELL_MAX_GROUPS = CELL_SCAN * 4 * CELL_THREADS;
 
 __global__ __launch_bounds__(CELL_THREADS) void k_comb_cells(
     Geo g, DevState *__restrict__ st, const int32_t *__restrict__ slot_tables, const SlotRec *__restrict__ slot_recs,
     int64_t ncap, int32_t *__restrict__ comb_tables, CombRec *__restrict__ comb_recs, int64_t ccap,
-    const int32_t *__restrict__ col_count, const int32_t *__restrict__ group, int gcols,
+    const int32_t *__restrict__ col_count, const int32_t *__restrict__ group, int ngroups, int gcols,
     const uint64_t *__restrict__ occ_bits, double *__restrict__ height) {
-    constexpr int COLS = 64 * CELL_PARTS, WAVES = CELL_THREADS / 64, PER = WAVES / CELL_PARTS;
-    __shared__ uint64_t occ[COLS * 4];
-    __shared__ uint32_t pre[COLS + 1];
-    __shared__ uint32_t part[WAVES];
+    constexpr int WAVES = CELL_THREADS / 64;
+    extern __shared__ uint4 first4[];   // first id of each group
+    uint32_t *first = reinterpret_cast<uint32_t *>(first4);
+    __shared__ uint32_t wtot[CELL_SCAN][WAVES];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int NW = (g.Z + 63) >> 6;
     const int32_t X = (int32_t)g.X;
     const int parity = st->parity, cur = 1 - parity, flip = st->flip;
     // origin of the combined map being built = newest slot's (gvom.py:229)
     const double *co = st->slot_origin[st->last_slot];
-    if (blockIdx.x == 0 && t == 0) begin_map(st, cur);
-    // part p of the block: the 64 columns from first_column(p) on
-    auto first_column = [&](int p) { return ((int32_t)blockIdx.x + p * (int32_t)gridDim.x) * 64; };
-    if (t < COLS) {
-        const int32_t c = first_column(w) + lane;
-        uint32_t n = 0;
-        for (int q = 0; q < NW; ++q) {
-            const uint64_t o = c < X ? occ_bits[(int64_t)c * NW + q] : 0ull;
-            occ[t * NW + q] = o;
-            n += __popcll(o);
+    uint4 v[CELL_SCAN];
+    const uint4 *g4 = reinterpret_cast<const uint4 *>(group);
+#pragma unroll
+    for (int q = 0; q < CELL_SCAN; ++q) {
+        // the last load may run past ngroups: the counts are padded
+        const int i = 4 * (q * CELL_THREADS + t);
+        v[q] = make_uint4(0, 0, 0, 0);
+        if (i < ngroups) {
+            v[q] = g4[i / 4];
+            if (i + 1 >= ngroups) v[q].y = 0;
+            if (i + 2 >= ngroups) v[q].z = 0;
+            if (i + 3 >= ngroups) v[q].w = 0;
         }
-        uint32_t v = n;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t u = __shfl_up(v, off);
-            if (lane >= off) v += u;
-        }
-        pre[t + 1] = v;
-        if (t == 0) pre[0] = 0;
     }
-    {
-        // first id of part w / PER, its terms shared by PER wavefronts
-        const int32_t c0 = first_column(w / PER);
-        const int at = (w % PER) * 64 + lane;
-        uint32_t base = 0;
-        if (c0 < X) {
-            const int32_t ng = c0 / gcols;
-            // four counts per load and several loads in flight (the last load may run past ng: the
-            // counts are padded)
-            const int4 *g4 = reinterpret_cast<const int4 *>(group);
-#pragma unroll 4
-            for (int32_t k = at; k < (ng + 3) / 4; k += 64 * PER) {
-                const int4 v = g4[k];
-                base += (uint32_t)v.x + (4 * k + 1 < ng ? (uint32_t)v.y : 0u) + (4 * k + 2 < ng ? (uint32_t)v.z : 0u) +
-                        (4 * k + 3 < ng ? (uint32_t)v.w : 0u);
-            }
-            for (int32_t c = ng * gcols + at; c < c0; c += 64 * PER) base += (uint32_t)col_count[c];
+    uint32_t before[CELL_SCAN];   // cells of the wavefront's groups before the thread's
+#pragma unroll
+    for (int q = 0; q < CELL_SCAN; ++q) {
+        if (q * 4 * CELL_THREADS >= ngroups) break;
+        const uint32_t n = v[q].x + v[q].y + v[q].z + v[q].w;
+        uint32_t p = n;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t u = __shfl_up(p, off);
+            if (lane >= off) p += u;
         }
-        for (int off = 32; off > 0; off >>= 1) base += __shfl_xor(base, off);
-        if (lane == 0) part[w] = base;
+        before[q] = p - n;
+        if (lane == 63) wtot[q][w] = p;
     }
     __syncthreads();
-    {
-        // prefixes within each part -> within the block
-        uint32_t add = 0;
-        if (t < COLS)
-            for (int q = 1; q <= w; ++q) add += pre[64 * q];
-        __syncthreads();
-        if (t < COLS) pre[t + 1] += add;
-        __syncthreads();
+    uint32_t n = 0;
+#pragma unroll
+    for (int q = 0; q < CELL_SCAN; ++q) {
+        if (q * 4 * CELL_THREADS >= ngroups) break;
+        uint32_t at = 0;
+#pragma unroll
+        for (int u = 0; u < WAVES; ++u) {
+            if (u == w) at = n;
+            n += wtot[q][u];
+        }
+        at += before[q];
+        const int i = q * CELL_THREADS + t;
+        if (4 * i < ngroups)
+            first4[i] = make_uint4(at, at + v[q].x, at + v[q].x + v[q].y, at + v[q].x + v[q].y + v[q].z);
     }
-    const uint32_t n = pre[COLS];
-    auto first_id = [&](int p) {   // minus the block's cells before the part
-        uint32_t v = part[p * PER];
-        for (int q = 1; q < PER; ++q) v += part[p * PER + q];
-        return v - pre[64 * p];
-    };
-    if (t < CELL_PARTS && first_column(t) < X && first_column(t) + 64 >= X) {
-        // the new map's cell count (the commit of gvom.py:276-316)
-        const int32_t total = (int32_t)(first_id(t) + pre[64 * (t + 1)]);
-        st->comb_cells[cur] = total;
-        st->comb_total = total;
+    __syncthreads();
+    if (blockIdx.x == 0 && t == 0) {
+        // the commit of gvom.py:276-316
+        begin_map(st, cur);
+        st->comb_cells[cur] = (int32_t)n;
+        st->comb_total = (int32_t)n;
     }
     CombRec *crec = comb_recs + (int64_t)cur * ccap;
     const CombRec *lrec = comb_recs + (int64_t)parity * ccap;
     int32_t *ctab = comb_tables + (int64_t)cur * g.V;
     const int32_t *ltab = comb_tables + (int64_t)parity * g.V;
-    for (uint32_t k = t; k < n; k += CELL_THREADS) {
-        // the cell's column: the last one whose first cell is at or before k
-        int cl = 0;
+    int top = 1;
+    while (4 * top < ngroups) top *= 4;
+    // 64 ids per wavefront, the blocks' first wavefronts first: few cells are spread over all blocks
+    for (uint32_t id = (w * gridDim.x + blockIdx.x) * 64 + lane; id < n; id += gridDim.x * CELL_THREADS) {
+        // the cell's group: the last one whose first id is at or before it
+        int gi = 0;
+        for (int step = top; step > 0; step >>= 2) {
+            int k = 0;
 #pragma unroll
-        for (int step = COLS / 2; step > 0; step >>= 1)
-            if (pre[cl + step] <= k) cl += step;
-        uint32_t r = k - pre[cl];
+            for (int u = 1; u < 4; ++u) k += gi + u * step < ngroups && first[min(gi + u * step, ngroups - 1)] <= id;
+            gi += k * step;
+        }
+        uint32_t r = id - first[gi];
+        // its column: the first one with more cells than r up to and including it (four counts per
+        // load, CELL_LOADS loads in flight; counts past the last column are never reached)
+        int32_t c = gi * gcols;
+        const uint4 *cc = reinterpret_cast<const uint4 *>(col_count + c);
+        uint32_t sum = 0, skip = 0;
+        int k = 0;
+        for (int q0 = 0; q0 < gcols / 4 && sum <= r; q0 += CELL_LOADS) {
+            uint4 m[CELL_LOADS];
+#pragma unroll
+            for (int u = 0; u < CELL_LOADS; ++u)
+                m[u] = q0 + u < gcols / 4 && c + 4 * (q0 + u) < X ? cc[q0 + u] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < CELL_LOADS; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    sum += j == 0 ? m[u].x : j == 1 ? m[u].y : j == 2 ? m[u].z : m[u].w;
+                    if (sum <= r) {
+                        skip = sum;
+                        k = 4 * (q0 + u) + j + 1;
+                    }
+                }
+        }
+        c += k;
+        r -= skip;
         const bool lowest = r == 0;
         int zw = 0;
-        uint64_t o = occ[cl * NW];
+        uint64_t o = occ_bits[(int64_t)c * NW];
         while (r >= (uint32_t)__popcll(o)) {
             r -= __popcll(o);
-            o = occ[cl * NW + ++zw];
+            o = occ_bits[(int64_t)c * NW + ++zw];
         }
         const int64_t z = zw * 64 + select_bit(o, (int)r);
-        const int64_t c = first_column(cl >> 6) + (cl & 63);
-        const int64_t lin = c * g.Z + z;
-        const uint32_t id = first_id(cl >> 6) + k;
+        const int64_t lin = (int64_t)c * g.Z + z;
         const uint32_t mask = (uint32_t)ctab[lin] & MASK31;
         ctab[lin] = (int32_t)(GVOM_OCC | id);
         CombRec out;
@@ -986,7 +1013,19 @@ int64_t zero_page_words() { return ZERO_PAGE_WORDS; }
 
 static int table_lanes(const Geo &g) { return (g.Z + ZPL - 1) / ZPL; }
 
-int64_t comb_group_columns(const Geo &g) { return 4 * (64 / table_lanes(g)); }
+// The table pass counts the occupied voxels per wavefront where the cell pass then has a count of
+// four columns or a multiple and at most four counts a thread to sum, per block otherwise.  Shorter
+// groups shorten a cell's walk, more of them lengthen the sum (cell pass, per block and per
+// wavefront): 64 x 64 x 32 (64 and 256 groups) 10.5 and 9.4 us, 128 x 128 x 32 13.2 and 11.4, 256 x
+// 256 x 8 18.8 and 14.9; but 256 x 256 x 64 (2048 and 8192) 16.9 and 18.5, 151 x 151 x 100 (1426 and
+// 5701) 11.1 and 12.5.
+constexpr int64_t WAVE_GROUPS = 4 * CELL_THREADS;
+static bool wave_groups(const Geo &g) {
+    const int cpw = 64 / table_lanes(g);
+    return cpw % 4 == 0 && (g.X + cpw - 1) / cpw <= WAVE_GROUPS;
+}
+
+int64_t comb_group_columns(const Geo &g) { return (wave_groups(g) ? 1 : 4) * (64 / table_lanes(g)); }
 int64_t comb_groups(const Geo &g) { return (g.X + comb_group_columns(g) - 1) / comb_group_columns(g); }
 
 hipError_t launch_comb_tables(const Geo &g, DevState *st, const int32_t *slot_tables, const int32_t *zero_page,
@@ -994,8 +1033,9 @@ hipError_t launch_comb_tables(const Geo &g, DevState *st, const int32_t *slot_ta
                               uint64_t *occ_bits, double *height, double *inferred, hipStream_t s) {
     if (comb_groups(g) > group_words) return hipErrorInvalidValue;
     const int zl = table_lanes(g);
-    k_comb_tables<<<(unsigned)comb_groups(g), 256, 0, s>>>(g, st, slot_tables, zero_page, comb_tables, col_count, group,
-                                                           occ_bits, height, inferred, zl, 64 / zl);
+    const int cpw = 64 / zl;
+    k_comb_tables<<<nblocks(g.X, 4 * cpw), 256, 0, s>>>(g, st, slot_tables, zero_page, comb_tables, col_count, group,
+                                                        occ_bits, height, inferred, zl, cpw, wave_groups(g));
     return hipGetLastError();
 }
 
@@ -1010,10 +1050,12 @@ hipError_t launch_scan_columns(int32_t *col_count, int64_t count_words, int64_t 
     return hipGetLastError();
 }
 
-// Maps of up to this many columns (256 x 256: one block of k_comb_cells per compute unit) merge
-// their cells there; larger ones run the column scan, k_comb_ids and k_comb_merge.  Measured
-// (rocprof, the kernels' sum): 65,536 columns 16.6 against 23.9 us, 22,801 11.5 against 18.9,
-// 4,096 8.1 against 15.2; but 102,400 columns 31 against 27, 160,000 55 against 47.
+// Maps of up to this many columns (256 x 256: CELL_MAX_GROUPS groups at the greatest height) merge
+// their cells in one kernel; larger ones run the column scan, k_comb_ids and k_comb_merge.  Measured
+// (rocprof, the kernels' sum, one kernel against three): 65,536 columns with 38k cells 16.9 against
+// 24.1 us, with 71k 20.0 against 32.1, with 71k of 30 slots 48 against 63; 22,801 columns 10.8
+// against 18.3, 4,096 9.4 against 15.2.  Past the line the one kernel would still be ahead where
+// its groups fit: 102,400 columns 21.8 against 33.8, 262,144 with 74k cells 26.2 against 38.5.
 constexpr int64_t CELL_MAX_COLUMNS = 65536;
 
 bool comb_cells_direct(const Geo &g) { return g.X <= CELL_MAX_COLUMNS; }
@@ -1023,10 +1065,12 @@ hipError_t launch_comb_cells(const Geo &g, DevState *st, const int32_t *slot_tab
                              int64_t count_words, const int32_t *group, int32_t *chunk_tot, int64_t chunk_words,
                              const uint64_t *occ_bits, uint2 *occ_list, double *height, hipStream_t s) {
     if (comb_cells_direct(g)) {
-        static_assert((CELL_PARTS & (CELL_PARTS - 1)) == 0 && CELL_THREADS % (64 * CELL_PARTS) == 0,
-                      "a thread per column, as many wavefronts per part");
-        k_comb_cells<<<nblocks((g.X + 63) / 64, CELL_PARTS), CELL_THREADS, 0, s>>>(
-            g, st, slot_tables, slot_recs, ncap, comb_tables, comb_recs, ccap, col_count, group,
+        const int64_t ng = comb_groups(g);
+        if (ng > CELL_MAX_GROUPS) return hipErrorInvalidValue;
+        static_assert(CELL_MAX_COLUMNS <= 8 * CELL_MAX_GROUPS, "groups have at least 8 columns (z_size 256)");
+        const unsigned nb = nblocks(g.V, CELL_THREADS);   // a small map's voxels need fewer blocks
+        k_comb_cells<<<nb < CELL_BLOCKS ? nb : CELL_BLOCKS, CELL_THREADS, (size_t)((ng + 3) / 4) * 16, s>>>(
+            g, st, slot_tables, slot_recs, ncap, comb_tables, comb_recs, ccap, col_count, group, (int)ng,
             (int)comb_group_columns(g), occ_bits, height);
         return hipGetLastError();
     }
