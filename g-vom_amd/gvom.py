@@ -306,7 +306,8 @@ class Gvom:
             return None
         out = np.empty((rows.value, 8), np.float32)
         nat.check(self._lib.gvom_debug_voxel_map(self._h, nat.ptr(out), rows.value, ctypes.byref(rows)), self._h)
-        return out
+        # a combine on another thread may have left fewer cells since the first call
+        return out[:rows.value]
 
     def make_debug_height_map(self):
         out = np.empty((self.xy_size * self.xy_size, 7), np.float32)
@@ -360,7 +361,8 @@ class Gvom:
         met = np.empty((C, 10), np.float64)
         nat.check(self._lib.gvom_get_slot(self._h, slot, nat.ptr(idx), C, nat.ptr(hit), nat.ptr(tot), nat.ptr(mh),
                                           nat.ptr(met), nat.ptr(origin), ctypes.byref(cells)), self._h)
-        return dict(index_map=idx, hit=hit, total=tot, min_h=mh, metrics=met, origin=origin)
+        C = cells.value   # another thread may have changed the slot since the first call
+        return dict(index_map=idx, hit=hit[:C], total=tot[:C], min_h=mh[:C], metrics=met[:C], origin=origin)
 
     def combined_state(self):
         cells = ctypes.c_int64(0)
@@ -379,7 +381,9 @@ class Gvom:
         nat.check(self._lib.gvom_get_combined(self._h, nat.ptr(idx), C, nat.ptr(hit), nat.ptr(tot), nat.ptr(mh),
                                               nat.ptr(met), nat.ptr(ev), nat.ptr(origin), ctypes.byref(cells)),
                   self._h)
-        return dict(index_map=idx, hit=hit, total=tot, min_h=mh, metrics=met, eigen=ev, origin=origin)
+        C = cells.value   # another thread may have combined since the first call
+        return dict(index_map=idx, hit=hit[:C], total=tot[:C], min_h=mh[:C], metrics=met[:C], eigen=ev[:C],
+                    origin=origin)
 
     def maps_state(self):
         X = self.xy_size
