@@ -2138,7 +2138,10 @@ extern "C" int gvom_autotune(gvom_handle *h, const void *points, int64_t n, int3
     int32_t *scratch = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int out = GVOM_OK;
-    int bb = h->ray_block, br = h->ray_rpt, bx = h->ray_box, bo = h->ray_xcd, bt = h->ray_tiled, ba = 0;
+    // the azimuth order is not used on scans below its line and not timed on one: kept as set then
+    const bool try_az = gvom_plan::az_pays(n, g.XY);
+    int bb = h->ray_block, br = h->ray_rpt, bx = h->ray_box, bo = h->ray_xcd, bt = h->ray_tiled;
+    int ba = try_az ? 0 : h->ray_az;
     float best = 1e30f;
     do {
         const bool can_tile = tiled_fits(g);
@@ -2203,7 +2206,6 @@ extern "C" int gvom_autotune(gvom_handle *h, const void *points, int64_t n, int3
                     }
                 }
         // the azimuth order, its grouping and the table clear included
-        const bool try_az = gvom_plan::az_pays(n, g.XY);
         if (out == GVOM_OK && try_az &&
             launch_prepare(dtype, points, h->world, h->k0, h->v0, h->valid, h->sd, 1, n, g, h->st, RAY_AZIMUTH, h->rsec,
                            nullptr, 0, h->azhist, h->azwords, st) != hipSuccess) {

@@ -197,7 +197,8 @@ class Gvom:
     def autotune(self, dev_points, n, ego_position, transform=None, dtype=np.float32):
         """Pick the ray-cast variant by timing it on one device-resident scan.  Returns
         (block, rays_per_thread, flags, best_ms); flags bit 0 LDS box, bit 1 sector order,
-        bit 2 tiled scratch, bit 3 spread (kept as set, not searched), bit 4 azimuth order."""
+        bit 2 tiled scratch, bit 3 spread (kept as set, not searched), bit 4 azimuth order (kept as
+        set by scans of fewer than 12e6 points x xy_size, which it does not take)."""
         ptr = dev_points.ptr if isinstance(dev_points, nat.DeviceArray) else ctypes.c_void_p(int(dev_points))
         ego = np.ascontiguousarray(np.asarray(ego_position, dtype=np.float64).reshape(3))
         T, tdt = _as_transform(transform)

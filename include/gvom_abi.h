@@ -323,7 +323,8 @@ void gvom_graph_destroy(gvom_graph *g);
  * and keeps the fastest.  chosen = {block, rays per thread, flags (bit 0 box, bit 1 sector
  * order, bit 2 tiled, bit 3 spread, bit 4 azimuth order)}; best_ms = its time.  The spread bit (wavefronts of a
  * block taken from across the scan) is not searched: it is kept as set, since it slows the
- * cast alone but speeds up a cast that overlaps a combine.  Synchronises. */
+ * cast alone but speeds up a cast that overlaps a combine.  So is the azimuth bit by a scan below
+ * the line, which that order does not take.  Synchronises. */
 int gvom_autotune(gvom_handle *h, const void *points, int64_t n, int32_t dtype, const double ego[3],
                   const void *T, int32_t t_dtype, int32_t chosen[3], float *best_ms);
 /* Sets the ray-cast configuration directly (flags as for gvom_autotune; the box and the
