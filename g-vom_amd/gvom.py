@@ -218,11 +218,18 @@ class Gvom:
         nat.check(self._lib.gvom_probe_atomics(self._h, int(pattern), int(n_atomics), out), self._h)
         return out[0], int(out[1])
 
-    def set_raycast_config(self, block=128, rays_per_thread=1, use_box=False, sector_order=False, tiled=True,
-                           spread=True, azimuth=False):
+    def set_raycast_config(self, block=128, rays_per_thread=1, use_box=None, sector_order=None, tiled=None,
+                           spread=True, azimuth=None):
         """Ray-cast launch shape and variant (tiled scratch excludes the LDS box; spread takes
-        each block's wavefronts from across the scan).  azimuth=True, as a new handle starts: scans
-        of at least 12e6 points x xy_size are cast in azimuth order, smaller ones as set here."""
+        each block's wavefronts from across the scan).  azimuth: scans of at least 12e6 points x
+        xy_size are cast in azimuth order, smaller ones as set here.  Without arguments, and for
+        those not given, as a new handle starts (tiled, spread, azimuth); but a call that chooses a
+        variant (use_box, sector_order or tiled, on or off) chooses it for scans of every size
+        unless it gives azimuth=True too."""
+        if azimuth is None:
+            azimuth = use_box is None and sector_order is None and tiled is None
+        if tiled is None:
+            tiled = True
         flags = ((1 if use_box else 0) | (2 if sector_order else 0) | (4 if tiled else 0) | (8 if spread else 0) |
                  (16 if azimuth else 0))
         nat.check(self._lib.gvom_set_raycast_config(self._h, int(block), int(rays_per_thread), flags), self._h)

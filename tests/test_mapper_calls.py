@@ -61,3 +61,21 @@ def test_state_of_a_map_that_shrinks_between_the_two_calls(name, rows):
     state = g.slot_state(0) if name == "slot_state" else g.combined_state()
     for k in rows:
         assert len(state[k]) == 3, k
+
+
+# flag bits: 1 LDS box, 2 sector order, 4 tiled scratch, 8 spread, 16 azimuth order
+@pytest.mark.parametrize("args,kw,expect", [
+    ((), {}, (128, 1, 4 + 8 + 16)),                                            # as a new handle starts
+    ((64,), {}, (64, 1, 4 + 8 + 16)),                                          # only the launch shape changes
+    ((), dict(rays_per_thread=2, spread=False), (128, 2, 4 + 16)),
+    ((256, 1, False, False, False, False), {}, (256, 1, 0)),                   # a variant for every scan
+    ((128, 1, False, False, True), {}, (128, 1, 4 + 8)),
+    ((256, 1), dict(use_box=True, tiled=False), (256, 1, 1 + 8)),
+    ((), dict(sector_order=True), (128, 1, 2 + 4 + 8)),
+    ((256, 1, False, False, False, False, True), {}, (256, 1, 16)),            # ... for the small ones
+    ((), dict(azimuth=False), (128, 1, 4 + 8)),
+])
+def test_raycast_config_flags(args, kw, expect):
+    g = _mapper(gvom_set_raycast_config=lambda h, *a: nat.GVOM_OK)
+    g.set_raycast_config(*args, **kw)
+    assert g._lib.calls == [("gvom_set_raycast_config", (None,) + expect)]
