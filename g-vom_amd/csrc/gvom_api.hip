@@ -14,7 +14,6 @@
 
 #include "gvom_kernels.h"
 
-hipError_t launch_clear_slots(int32_t *slot_tables, const DevState *st, int S, const Geo &g, hipStream_t s);
 int64_t diff_partials(int64_t n_points, int64_t X, int64_t ncap);
 int64_t diff_rec_bytes();
 hipError_t launch_diff_forward(const Geo &g, const DevState *st, int slot, const int32_t *table,
@@ -150,6 +149,7 @@ struct gvom_handle {
     int32_t *zero_page = nullptr;   // zeros the combine reads in place of off-map words
     uint2 *occ_list = nullptr;        // compact cell list (large maps only)
     int32_t *group_count = nullptr;   // occupied voxels per group of columns of the combined map
+    int64_t group_words = 0;
     int32_t *export_buf = nullptr;
     int32_t *chunk_tot = nullptr;
 
@@ -448,7 +448,8 @@ extern "C" int gvom_create(const gvom_params *params, gvom_handle **out) {
     h->rough = (double *)(h->vis + X);
     CKC(dalloc(&h->delta, X));
     if (!comb_cells_direct(g)) CKC(dalloc(&h->occ_list, V));
-    CKC(dalloc(&h->group_count, comb_groups(g) + 3));   // read four at a time
+    h->group_words = comb_group_words(g);
+    CKC(dalloc(&h->group_count, h->group_words));
     h->col_count_words = gvom_plan::alloc_col_count_words(X);
     CKC(dalloc(&h->col_count, h->col_count_words));
     CKC(dalloc(&h->occ_bits, X * ((g.Z + 63) / 64)));
@@ -914,7 +915,7 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     // the direct casts count into cleared tables; on one stream the sort's first pass, which leaves
     // most of the chip idle, clears them
     const bool own_clear = !az && !tiled && (fork || NT <= 0);
-    const SlotClear clear{h->slot_tables, g.B, S, g.V};
+    const SlotClear clear{h->slot_tables, h->slot_table_words, g.B, S, g.V};
     CKH(h, radix_sort(W.k0, W.v0, W.k1, W.v1, NT, g.VB + sbits, g.VB, W.hist, W.hwords, h->st, &sk, &sv, cs,
                       !az && !tiled && !own_clear ? &clear : nullptr));
     h->sorted_vals = sv;
@@ -926,7 +927,7 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
     if (az)
         CKH(h, launch_az_order(W.rsec, W.valid, sd, S, NT, g, h->st, W.azhist, W.azwords, W.rorder, h->slot_tables,
                                h->slot_table_words, -1, fs));
-    else if (own_clear) CKH(h, launch_clear_slots(h->slot_tables, h->st, S, g, fs));
+    else if (own_clear) CKH(h, launch_clear_slots(h->slot_tables, h->slot_table_words, h->st, S, g, fs));
     stage_event(h, 1, fs);
     if (az)
         CKH(h, launch_raycast_az(dtype, W.world, sd, S, NT, g, h->st, h->slot_tables, h->slot_table_words, W.rorder,
@@ -1273,12 +1274,12 @@ static int combine_impl(gvom_handle *h, uint8_t *host_maps = nullptr) {
     const int cur = 1 - h->parity;
     stage_event(h, 5);
     CKH(h, launch_comb_tables(g, h->st, h->slot_tables, h->zero_page, h->comb_tables, h->col_count, h->group_count,
-                              comb_groups(g), h->occ_bits, h->height, h->inferred, st));
+                              h->group_words, h->occ_bits, h->height, h->inferred, st));
     stage_event(h, 6);
     CKH(h, join_metrics(h));   // the record merge reads the newest stage's metrics
     CKH(h, launch_comb_cells(g, h->st, h->slot_tables, h->slot_recs, h->ncap, h->comb_tables, h->comb_recs, h->ccap,
-                             h->col_count, h->col_count_words, h->group_count, h->chunk_tot, h->chunk_tot_words,
-                             h->occ_bits, h->occ_list, h->height, st));
+                             h->col_count, h->col_count_words, h->group_count, h->group_words, h->chunk_tot,
+                             h->chunk_tot_words, h->occ_bits, h->occ_list, h->height, st));
     stage_event(h, 7);
     CKH(h, launch_maps2d(g, h->st, h->height, h->inferred, h->comb_tables, h->comb_recs, h->ccap, h->slope_x,
                          h->slope_y, h->rough, h->delta, h->pos, h->neg, h->vis, host_maps, st));

@@ -53,6 +53,7 @@ constexpr int ZPL = 8;           // voxels per lane
 constexpr int SRC_GROUP = 4;     // sources loaded together
 constexpr int ZERO_PAGE_WORDS = 64;
 static_assert(ZPL == 8, "two 16-byte loads, one byte of occupancy bits per lane");
+static_assert(ZPL - 1 <= TABLE_PAD && ZPL <= ZERO_PAGE_WORDS, "a lane's loads stay inside the padded tables");
 
 // four words at a 4-byte aligned address
 typedef int32_t words4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -1027,11 +1028,12 @@ static bool wave_groups(const Geo &g) {
 
 int64_t comb_group_columns(const Geo &g) { return (wave_groups(g) ? 1 : 4) * (64 / table_lanes(g)); }
 int64_t comb_groups(const Geo &g) { return (g.X + comb_group_columns(g) - 1) / comb_group_columns(g); }
+int64_t comb_group_words(const Geo &g) { return (comb_groups(g) + 3) / 4 * 4; }
 
 hipError_t launch_comb_tables(const Geo &g, DevState *st, const int32_t *slot_tables, const int32_t *zero_page,
                               int32_t *comb_tables, int32_t *col_count, int32_t *group, int64_t group_words,
                               uint64_t *occ_bits, double *height, double *inferred, hipStream_t s) {
-    if (comb_groups(g) > group_words) return hipErrorInvalidValue;
+    if (comb_group_words(g) > group_words) return hipErrorInvalidValue;
     const int zl = table_lanes(g);
     const int cpw = 64 / zl;
     k_comb_tables<<<nblocks(g.X, 4 * cpw), 256, 0, s>>>(g, st, slot_tables, zero_page, comb_tables, col_count, group,
@@ -1062,12 +1064,15 @@ bool comb_cells_direct(const Geo &g) { return g.X <= CELL_MAX_COLUMNS; }
 
 hipError_t launch_comb_cells(const Geo &g, DevState *st, const int32_t *slot_tables, const SlotRec *slot_recs,
                              int64_t ncap, int32_t *comb_tables, CombRec *comb_recs, int64_t ccap, int32_t *col_count,
-                             int64_t count_words, const int32_t *group, int32_t *chunk_tot, int64_t chunk_words,
-                             const uint64_t *occ_bits, uint2 *occ_list, double *height, hipStream_t s) {
+                             int64_t count_words, const int32_t *group, int64_t group_words, int32_t *chunk_tot,
+                             int64_t chunk_words, const uint64_t *occ_bits, uint2 *occ_list, double *height,
+                             hipStream_t s) {
     if (comb_cells_direct(g)) {
         const int64_t ng = comb_groups(g);
-        if (ng > CELL_MAX_GROUPS) return hipErrorInvalidValue;
-        static_assert(CELL_MAX_COLUMNS <= 8 * CELL_MAX_GROUPS, "groups have at least 8 columns (z_size 256)");
+        // the last column counts are read four at a time as well
+        if (ng > CELL_MAX_GROUPS || comb_group_words(g) > group_words || (g.X + 3) / 4 * 4 > count_words)
+            return hipErrorInvalidValue;
+        static_assert(CELL_MAX_COLUMNS <= 8 * CELL_MAX_GROUPS, "groups past WAVE_GROUPS have at least 8 columns (z_size 256)");
         const unsigned nb = nblocks(g.V, CELL_THREADS);   // a small map's voxels need fewer blocks
         k_comb_cells<<<nb < CELL_BLOCKS ? nb : CELL_BLOCKS, CELL_THREADS, (size_t)((ng + 3) / 4) * 16, s>>>(
             g, st, slot_tables, slot_recs, ncap, comb_tables, comb_recs, ccap, col_count, group, (int)ng,

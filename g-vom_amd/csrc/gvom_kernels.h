@@ -55,9 +55,11 @@ hipError_t launch_raycast(int dtype, const void *world, const uint8_t *valid, co
 // buffer pair holds the result.
 // scan_shift: keys >> scan_shift is the scan of the batch (the first pass counts each scan's
 // valid keys into set 1).
-// The S slot tables of V words a scan stage counts into, cleared by the first pass of its sort.
+// The S slot tables of V words a scan stage counts into (of `words` words of tables in all), cleared
+// by the first pass of its sort.
 struct SlotClear {
     int32_t *tables;
+    int64_t words;
     int B, S;
     int64_t V;
 };
@@ -66,6 +68,9 @@ hipError_t radix_sort(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, in
                       hipStream_t s,
                       const SlotClear *clear = nullptr);
 int64_t radix_hist_entries(int64_t n);
+// The same clear as a launch of its own (table_words: words of slot_tables).
+hipError_t launch_clear_slots(int32_t *slot_tables, int64_t table_words, const DevState *st, int S, const Geo &g,
+                              hipStream_t s);
 // words of the segment kernels' per-block counts (launch_segments' blk) for n sorted keys
 int64_t segment_block_words(int64_t n);
 // Segments of equal keys in the sorted array, per-scan bounds and slot cell counts, and the
@@ -97,9 +102,11 @@ hipError_t launch_commit_process(DevState *st, const ScanDesc *sd, const Geo &g,
 // comb_tables must be readable for TABLE_PAD words before and after.
 constexpr int64_t TABLE_PAD = 64;
 int64_t zero_page_words();
-// group: occupied voxels per group of comb_group_columns(g) consecutive columns.
+// group: occupied voxels per group of comb_group_columns(g) consecutive columns, comb_groups(g)
+// counts in comb_group_words(g) words (the cell pass reads four at a time).
 int64_t comb_group_columns(const Geo &g);
 int64_t comb_groups(const Geo &g);
+int64_t comb_group_words(const Geo &g);
 hipError_t launch_comb_tables(const Geo &g, DevState *st, const int32_t *slot_tables, const int32_t *zero_page,
                               int32_t *comb_tables, int32_t *col_count, int32_t *group, int64_t group_words,
                               uint64_t *occ_bits, double *height, double *inferred, hipStream_t s);
@@ -112,8 +119,9 @@ hipError_t launch_scan_columns(int32_t *col_count, int64_t count_words, int64_t 
 bool comb_cells_direct(const Geo &g);
 hipError_t launch_comb_cells(const Geo &g, DevState *st, const int32_t *slot_tables, const SlotRec *slot_recs,
                              int64_t ncap, int32_t *comb_tables, CombRec *comb_recs, int64_t ccap, int32_t *col_count,
-                             int64_t count_words, const int32_t *group, int32_t *chunk_tot, int64_t chunk_words,
-                             const uint64_t *occ_bits, uint2 *occ_list, double *height, hipStream_t s);
+                             int64_t count_words, const int32_t *group, int64_t group_words, int32_t *chunk_tot,
+                             int64_t chunk_words, const uint64_t *occ_bits, uint2 *occ_list, double *height,
+                             hipStream_t s);
 hipError_t launch_maps2d(const Geo &g, DevState *st, const double *height, const double *inferred,
                          const int32_t *comb_tables, const CombRec *comb_recs, int64_t ccap, double *slope_x,
                          double *slope_y, double *rough, double *delta, int32_t *pos, int32_t *neg, int32_t *vis,

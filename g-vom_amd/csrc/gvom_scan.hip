@@ -617,11 +617,13 @@ static_assert(AZ_SEG % AZ_BATCH == 0, "whole batches");
 // LDS counters per block: the wedges' need for a scan of n rays on this map (rows of 1 + d dt
 // columns, dt = 2 x the wedge's angle on the diagonals, of about 3/4 of the heights), at most
 // 48 KiB, so that two blocks and a sort block of the other stream fit a compute unit's 160 KiB.
+constexpr int64_t AZ_COUNTERS = 24576;
+static_assert(AZ_COUNTERS % 1024 == 0 && AZ_COUNTERS < 32768, "a counter's place: exact as a float with a half");
 inline int64_t az_lds_counters(const Geo &g, int64_t n) {
     const double half = g.XY / 2.0 < AZ_DIST ? g.XY / 2.0 : AZ_DIST;
     const double dt = 2.0 * 6.2832 * AZ_RAYS / (double)(n > AZ_RAYS ? n : AZ_RAYS);
     const double need = (half + 0.5 * half * half * dt) * g.Z * 0.75;
-    int64_t c = need < 24576.0 ? (int64_t)need : 24576;
+    int64_t c = need < (double)AZ_COUNTERS ? (int64_t)need : AZ_COUNTERS;
     c = (c + 1023) / 1024 * 1024;
     return c < 4096 ? 4096 : c;
 }
@@ -2120,6 +2122,9 @@ hipError_t radix_sort(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, in
     auto status = [&](int p) { return hist + (int64_t)p * hwords; };
     auto totals = [&](int p) { return hist + (int64_t)p * hwords + gvom_plan::radix_totals_at(n); };
     uint32_t *ka = k0, *va = v0, *kb = k1, *vb = v1;
+    if (clear && (clear->S < 1 || clear->S > GVOM_MAX_BATCH ||
+                  gvom_plan::slot_table_footprint(clear->V, clear->B, -1) > clear->words))
+        return hipErrorInvalidValue;
     for (int p = 0; p < passes; ++p) {
         uint32_t *tn = p + 1 < passes ? totals(p + 1) : nullptr;
         if (p == 0) {
@@ -2199,7 +2204,10 @@ hipError_t launch_commit_process(DevState *st, const ScanDesc *sd, const Geo &g,
     return hipGetLastError();
 }
 
-hipError_t launch_clear_slots(int32_t *slot_tables, const DevState *st, int S, const Geo &g, hipStream_t s) {
+hipError_t launch_clear_slots(int32_t *slot_tables, int64_t table_words, const DevState *st, int S, const Geo &g,
+                              hipStream_t s) {
+    if (S < 1 || S > GVOM_MAX_BATCH || gvom_plan::slot_table_footprint(g.V, g.B, -1) > table_words)
+        return hipErrorInvalidValue;
     k_clear_slots<<<dim3((unsigned)((g.V + 4095) / 4096), (unsigned)S), 256, 0, s>>>(slot_tables, st, g.B,
                                                                                     (int32_t)g.V);
     return hipGetLastError();
