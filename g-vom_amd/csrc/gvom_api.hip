@@ -503,6 +503,8 @@ static int ensure_capacity(gvom_handle *h, int64_t max_scan, int64_t batch_pts) 
     }
     int64_t need_ncap = max_scan < g.V ? max_scan : g.V;
     if (need_ncap < 1) need_ncap = 1;
+    // an overlapped stage's metrics may still write the records and read the work buffers moved below
+    if (need_ncap > h->ncap || batch_pts > h->ptcap) CKH(h, join_metrics(h));
     if (need_ncap > h->ncap) {
         int64_t nc = h->ncap * 2 > need_ncap ? h->ncap * 2 : need_ncap;
         if (nc > g.V) nc = g.V;
