@@ -350,7 +350,11 @@ static hipError_t dalloc(T **p, int64_t count) {
 
 // Events that only order the handle's streams on its own device, never waited for by the host:
 // no release to system scope where they are recorded (five or six a frame: 131,072 points on 256 x
-// 256 x 64 145.4 -> 140.4 us, with overlap 146.5 -> 137.8).
+// 256 x 64 145.4 -> 140.4 us, with overlap 146.5 -> 137.8).  What this rests on, and has to hold at
+// every recording: the device memory that the waiting stream reads was last written by kernels,
+// which end with a release to the whole device (its eight L2s among them), or by a copy or fill
+// that the host has waited for since; and host memory written before such an event is read by the
+// host only after it has waited for the main stream itself.
 constexpr unsigned ORDER_EVENT = hipEventDisableTiming | hipEventDisableSystemFence;
 
 extern "C" int gvom_create(const gvom_params *params, gvom_handle **out) {
@@ -643,7 +647,7 @@ static int ensure_tile_scratch(gvom_handle *h) {
     }
     CKH(h, dalloc(&h->tscratch, words * n));
     ++h->buf_gen;
-    CKH(h, hipMemsetAsync(h->tscratch, 0, (size_t)words * n * sizeof(int32_t), h->stream));
+    CKH(h, launch_fill_i32(h->tscratch, 0, words * n, h->stream));
     CKH(h, mark_back(h));
     h->tscratch_scans = n;
     h->tscratch_words = words * n;
