@@ -233,6 +233,7 @@ struct gvom_handle {
     // azimuth-ordered cast for scans it pays for (gvom_plan::az_pays); the settings below apply
     // to the others, or to all when it is off
     int ray_az = 1;
+    int last_cast = 0, hp_cast = 0;   // gvom_last_cast; that of the replayed sequence
     int ray_block = 128, ray_rpt = 1, ray_box = 0, ray_xcd = 0, ray_spread = 1;
     int64_t ray_stride = 0;   // gvom_set_ray_rings: points per ring (0: linear ray order)
     int ray_patch = 0;        // rings per patch
@@ -891,6 +892,7 @@ static int process_impl(gvom_handle *h, const void *xyz, const int64_t *offsets,
         CKH(h, launch_set_descs(h->sd, sdh, S, fs));
     }
     h->diff_n = -1;   // every check passed: the work buffers a pending gvom_diff_backward reads are reused below
+    h->last_cast = az ? 3 : tiled ? 2 : cast ? 1 : 0;
     stage_event(h, 0, fs);
     const bool xcd = cast && !az && h->ray_xcd != 0;
     if (xcd) CKH(h, launch_fill_i32(&h->st->sec_count[0], 0, 16, fs));   // sec_count and sec_cursor
@@ -1076,6 +1078,7 @@ static void capture_host_process(gvom_handle *h, int64_t n, int dtype, const dou
         return;
     }
     h->hp_n = n;
+    h->hp_cast = h->last_cast;
     h->hp_dtype = dtype;
     h->hp_src = src;
     h->hp_gen = gen;
@@ -1133,6 +1136,7 @@ static int process_host_replay(gvom_handle *h, const void *xyz, int64_t n, int d
     std::memcpy((uint8_t *)h->pin_pts[k] + off, &d, sizeof(d));
     h->diff_n = -1;   // the sequence reuses the work buffers a pending gvom_diff_backward reads
     CKH(h, hipGraphLaunch(h->hp_exec[k], h->stream));
+    h->last_cast = h->hp_cast;
     CKH(h, hipEventRecord(h->ev_pin[k], h->stream));
     h->pin_next = 1 - k;
     CKH(h, mark_back(h));
@@ -2297,6 +2301,12 @@ extern "C" int gvom_set_overlap(gvom_handle *h, int32_t enabled) {
     }
     h->overlap = enabled ? 1 : 0;
     ++h->cfg_gen;
+    return GVOM_OK;
+}
+
+extern "C" int gvom_last_cast(const gvom_handle *h, int32_t *cast) {
+    if (!h || !cast) return GVOM_EINVAL;
+    *cast = h->last_cast;
     return GVOM_OK;
 }
 

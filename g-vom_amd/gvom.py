@@ -234,6 +234,12 @@ class Gvom:
                  (16 if azimuth else 0))
         nat.check(self._lib.gvom_set_raycast_config(self._h, int(block), int(rays_per_thread), flags), self._h)
 
+    def last_cast(self):
+        """The cast of the last scan stage: "none", "direct", "tiled" or "azimuth"."""
+        cast = ctypes.c_int32()
+        nat.check(self._lib.gvom_last_cast(self._h, ctypes.byref(cast)), self._h)
+        return ("none", "direct", "tiled", "azimuth")[cast.value]
+
     def set_ray_rings(self, points_per_ring, patch_rings=32):
         """Ray order hint for organised scans (rings of points_per_ring consecutive points):
         each wavefront of the ray cast traces 64 / patch_rings azimuths x patch_rings rings.

@@ -335,6 +335,11 @@ int gvom_autotune(gvom_handle *h, const void *points, int64_t n, int32_t dtype, 
  * process call that uses it, gvom_reserve or gvom_graph_begin. */
 int gvom_set_raycast_config(gvom_handle *h, int32_t block, int32_t rays_per_thread, int32_t flags);
 
+/* The cast of the scan stage last issued (or recorded, inside a capture) by a process call: 0 none
+ * yet or a stage without a cast, 1 into the slot tables, 2 through the tiled scratch, 3 in azimuth
+ * order (diagnostics: every cast leaves the same counts). */
+int gvom_last_cast(const gvom_handle *h, int32_t *cast);
+
 /* Ray order hint (no reference counterpart): the scans are organised in rings of
  * points_per_ring consecutive points (a spinning lidar's PointCloud2 rows, e.g. 1024 for a
  * 1024-azimuth sensor).  Each wavefront of the ray cast then traces a patch of
