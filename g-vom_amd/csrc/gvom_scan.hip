@@ -587,8 +587,9 @@ __global__ __launch_bounds__(256) void k_raycast(const P *__restrict__ world,
 // other axis or z, a rounded edge, rows past the counters' room) updates the slot table
 // directly: the layout decides only where a step is counted.
 //
-// Counters are 16 bits, two to a word: a ray enters a voxel at most once (its dominant
-// coordinate moves one voxel a step), so a counter holds at most AZ_RAYS.
+// Counters are 16 bits, two to a word.  A ray's dominant coordinate moves one voxel a step, but on
+// the way down past a power of two the f32 sum may round back onto the integer it should leave:
+// a ray counts in a voxel at most twice, a counter holds at most 2 AZ_RAYS.
 //
 // A step is a chain of dependent instructions, so a ray's steps are dealt to several lanes: an
 // item is up to `seg` consecutive steps of one ray, and its lane first repeats the f32
@@ -610,7 +611,7 @@ constexpr int AZ_DIST = 512;      // rows of the LDS layout
 constexpr int AZ_SEGS = 16;       // most items of one ray
 constexpr int AZ_SEG = 32;        // steps per item, doubled until AZ_SEGS items hold the longest ray
 constexpr int AZ_BATCH = 4;       // steps whose layout rows are read together
-static_assert(AZ_RAYS == 256 && AZ_THREADS == 2 * AZ_RAYS && AZ_DIST == AZ_THREADS,
+static_assert(AZ_RAYS == 256 && AZ_THREADS == 2 * AZ_RAYS && AZ_DIST == AZ_THREADS && 2 * AZ_RAYS < 65536,
               "item = ray | segment << 8; one row a thread; 16-bit counters");
 static_assert(AZ_SEG % AZ_BATCH == 0, "whole batches");
 
