@@ -21,6 +21,7 @@
 //             count, written by the cell pass.
 #include <hip/hip_runtime.h>
 
+#include "gvom_cell_walk.h"
 #include "gvom_kernels.h"
 
 
@@ -462,7 +463,6 @@ __device__ __forceinline__ void merge_cell(const Geo &g, const DevState *__restr
 // above, 1024 30.5 and 19.0, 256 blocks of four 30.5 and 18.2.
 constexpr int CELL_THREADS = 512;
 constexpr int CELL_SCAN = 4;      // prefix sum: up to CELL_SCAN x 4 groups per thread
-constexpr int CELL_LOADS = 4;     // 16 in flight: 0.4 to 0.9 us longer
 constexpr int CELL_BLOCKS = 256;
 constexpr int CELL_MAX_GROUPS = CELL_SCAN * 4 * CELL_THREADS;
 
@@ -548,30 +548,8 @@ __global__ __launch_bounds__(CELL_THREADS) void k_comb_cells(
             gi += k * step;
         }
         uint32_t r = id - first[gi];
-        // its column: the first one with more cells than r up to and including it (four counts per
-        // load, CELL_LOADS loads in flight; counts past the last column are never reached)
         int32_t c = gi * gcols;
-        const uint4 *cc = reinterpret_cast<const uint4 *>(col_count + c);
-        uint32_t sum = 0, skip = 0;
-        int k = 0;
-        for (int q0 = 0; q0 < gcols / 4 && sum <= r; q0 += CELL_LOADS) {
-            uint4 m[CELL_LOADS];
-#pragma unroll
-            for (int u = 0; u < CELL_LOADS; ++u)
-                m[u] = q0 + u < gcols / 4 && c + 4 * (q0 + u) < X ? cc[q0 + u] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int u = 0; u < CELL_LOADS; ++u)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    sum += j == 0 ? m[u].x : j == 1 ? m[u].y : j == 2 ? m[u].z : m[u].w;
-                    if (sum <= r) {
-                        skip = sum;
-                        k = 4 * (q0 + u) + j + 1;
-                    }
-                }
-        }
-        c += k;
-        r -= skip;
+        c += cell_column(reinterpret_cast<const uint4 *>(col_count + c), gcols, X - c, r);
         const bool lowest = r == 0;
         int zw = 0;
         uint64_t o = occ_bits[(int64_t)c * NW];
